@@ -1,4 +1,4 @@
-"""Generates the block loop of ``bwd_dkdv_wide_kernel`` as gfx950 assembly.
+"""Generates the block loop of ``dkdv_wide`` as gfx950 assembly.
 
 The arithmetic is the dK / dV part of the derivative of the reference branch
 kernel (swiattn_gqa_prefill_varlen.py V:176-241; the reference itself is
@@ -553,7 +553,7 @@ def epilogue():
     """dK = scale dK^T and dV = dV^T as bf16 rows, four values per store, at
     each lane's key row (keys past the end fall outside the descriptors); or,
     for one split of a pair's row blocks, the fp32 partials for
-    bwd_dkdv_reduce_kernel: key half kh of the wave is the reduce's wave
+    bwd_reduce_kernel: key half kh of the wave is the reduce's wave
     2 w + kh, dK^T block db elements 4 j .. 4 j + 3 its unit 4 db + j (with
     the sign of dS^T Q: the loop accumulated its negative) and dV^T's unit
     16 + 4 db + j, at (32 kh + unit) KiB + 16 lane of the wave's part.
@@ -666,7 +666,7 @@ def clobbers():
 def emit(path):
     lines = generate()
     with open(path, "w") as f:
-        f.write("// Generated by gen_bwd_dkdv.py: the block loop of bwd_dkdv_wide_kernel.  Do not edit.\n")
+        f.write("// Generated by gen_bwd_dkdv.py: the block loop of dkdv_wide.  Do not edit.\n")
         f.write("#pragma once\n")
         f.write("#define SWATTN_BWD_DKDV_ASM \\\n")
         for ln in lines:

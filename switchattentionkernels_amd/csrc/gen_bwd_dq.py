@@ -1,4 +1,4 @@
-"""Generates the tile loop of ``bwd_dq_wide_kernel`` as gfx950 assembly.
+"""Generates the tile loop of ``dq_wide`` as gfx950 assembly.
 
 The arithmetic is the dQ part of the derivative of the reference branch
 kernel (swiattn_gqa_prefill_varlen.py V:176-241; the reference itself is
@@ -586,7 +586,7 @@ def clobbers():
 def emit(path):
     lines = generate()
     with open(path, "w") as f:
-        f.write("// Generated by gen_bwd_dq.py: the tile loop of bwd_dq_wide_kernel.  Do not edit.\n")
+        f.write("// Generated by gen_bwd_dq.py: the tile loop of dq_wide.  Do not edit.\n")
         f.write("#pragma once\n")
         f.write("#define SWATTN_BWD_DQ_ASM \\\n")
         for ln in lines:

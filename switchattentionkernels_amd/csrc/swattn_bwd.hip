@@ -23,7 +23,7 @@
 //   operands in registers and dK^T, dV^T (128 d x 32 keys each) in
 //   accumulators; the workgroup's V rows sit in LDS.  It streams the row
 //   blocks that can see the tile (a contiguous block range per branch,
-//   found by bwd_ranges_kernel with a wave-parallel search over the
+//   found by bwd_prep_kernel with a wave-parallel search over the
 //   monotone row bounds) through a three-slot LDS ring.  Each block's 32 Q and dO rows
 //   are gathered from their positions by global_load_lds_dwordx4 (one
 //   64-bit source address per lane), from the row offsets of the block's
@@ -43,14 +43,16 @@
 // * Keys outside a row's range get S = -inf, so P = 0 exactly; a row with no
 //   legal key (or a padding row) carries LSE = Delta = 0 and bounds [0, 0),
 //   is masked everywhere and contributes nothing.
-// * Grids of fewer than 512 (key tile, KV head) pairs split each pair over
-//   its row blocks (up to 16 workgroups); bwd_dkdv_reduce_kernel sums the
-//   fp32 partials in split order.  Pairs run longest first (the first key
-//   tiles of each sequence are seen by the most rows).  When the longest
-//   dQ row tile (the latest full rows see every earlier key) would set the
-//   dQ kernel's length, row tiles longer than the estimated key tiles per
-//   workgroup slot are cut into equal pieces of their key range; pieces
-//   write fp32 partials that bwd_dq_reduce_kernel sums in piece order.
+// * Both products run in one grid (bwd_wide_kernel), dK/dV's workgroups first:
+//   dQ's fill the CUs that dK/dV's leave, and small grids run both at once.
+//   Grids of fewer than 512 (key tile, KV head) pairs may cut a pair over its
+//   row blocks (up to 16 workgroups) where it would outlast the grid's time per
+//   CU.  Pairs run longest first (the first key tiles of each sequence are seen
+//   by the most rows).  When the longest dQ row tile (the latest full rows see
+//   every earlier key) would set dQ's length, row tiles longer than the
+//   estimated key tiles per workgroup slot are cut into equal pieces of their
+//   key range.  Cut workgroups write fp32 partials that bwd_reduce_kernel sums
+//   in their order.
 // * dQ is a separate pass (S and dP recomputed) rather than atomics from the
 //   key-stationary pass, so every output is written once, deterministically.
 
@@ -95,10 +97,11 @@ constexpr int kDkvLdsBytes = kVTileBytes + kRingSlots * kStageBytes + kInfoSlots
 constexpr int kPartUnits = 32;
 constexpr size_t kPartBytesPerWg = static_cast<size_t>(kBwdWaves) * kPartUnits * 64 * 16;   // 256 KiB
 // Below this many dK/dV workgroups (two rounds of one per CU on a 256-CU
-// MI355X: the kernel's LDS allows one) the (key tile, KV head) pairs are
-// split over their row blocks.
+// MI355X: the kernel's LDS allows one) the workspace has room to cut the (key
+// tile, KV head) pairs over their row blocks.
 constexpr int64_t kDkvTargetWgs = 512;
 constexpr int kDkvMaxSplit = 16;
+constexpr int64_t kDkvMinBlocks = 4;   // row blocks a cut pair's share takes at least
 // dQ workgroups that run at once (one per CU: the 96 KiB ring allows one).
 constexpr int64_t kDqSlots = 256;
 // dQ piece partials: per workgroup and wave, 16 float4 units per lane (dQ^T
@@ -131,7 +134,10 @@ struct BwdParams {
   uint16_t* zero_row;        // 128 zeros: the gather source of rows that contribute nothing
   int32_t* ranges;           // [2][kv_tiles_dkv][2] block ranges
   float* dkv_part;           // dK/dV split partials (dkv_split > 1): [workgroup][8 waves][32][64 lanes] float4
-  int32_t dkv_split;         // dK/dV workgroups per (key tile, KV head), over its row blocks
+  int32_t dkv_split;         // dK/dV workgroup slots per (key tile, KV head)
+  int32_t dkv_chunk;         // row blocks per dK/dV workgroup (a pair is cut into at most dkv_split)
+  int32_t dkv_wgs;           // bwd_wide_kernel: workgroups below this are dK/dV's, the rest dQ's
+  int32_t prep_wgs;          // bwd_prep_kernel: workgroups below this prepare blocks, the rest ranges
   int32_t dkv_batches;       // > 1: key tiles ordered tile-in-sequence-major over this many sequences
   float* dq_part;            // dQ piece partials (dq_chunk > 0): [workgroup][8 waves][16][64 lanes] float4
   int32_t* dq_nch;           // pieces per (row tile, KV head), written by piece 0 (dq_chunk > 0)
@@ -168,7 +174,7 @@ __device__ __forceinline__ void row_bounds(const BwdParams& p, int branch, int p
   // An empty range keeps ks = ke.  F's rule with seq_q > seq_kv + window - 1
   // gives late local rows a start past their end (and past the next
   // sequence's first start); clipped, the starts are non-decreasing along
-  // each list, as bwd_ranges_kernel's search needs.
+  // each list, as the search of block_ranges needs.
   ks = min(ks, ke);
 }
 
@@ -183,9 +189,10 @@ __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w 
 // Preparation: one workgroup per (branch, block of 32 rows, KV head).
 // ---------------------------------------------------------------------------
 template <bool kMeta>
-__global__ __launch_bounds__(kThreads) void bwd_prep_kernel(const BwdParams p) {
+__device__ __forceinline__ void prep_block(const BwdParams& p, int wg) {
   __shared__ int s_ks[kBRows], s_ke[kBRows];
-  const int x = blockIdx.x, kvh = blockIdx.y;
+  const int nblk = p.blocks[0] + p.blocks[1];
+  const int kvh = wg / nblk, x = wg - kvh * nblk;
   const int b = x < p.blocks[0] ? 0 : 1;
   const int blk = x - (b ? p.blocks[0] : 0);
   const int64_t pb = packed_block(p, b, kvh, blk);
@@ -243,7 +250,7 @@ __global__ __launch_bounds__(kThreads) void bwd_prep_kernel(const BwdParams p) {
     infi[kInfoStart + rr] = live ? ks : 0;
     infi[kInfoEnd + rr] = live ? ke : 0;
     reinterpret_cast<int64_t*>(inf)[kInfoRowOff + rr] = live ? row_off : -1;
-    // The same as a 32-bit byte offset for bwd_dkdv_wide_kernel's buffer
+    // The same as a 32-bit byte offset for dkdv_wide's buffer
     // loads (only used where Q is below 2^31 bytes; past every range when
     // the row contributes nothing, so that its loads read zeros).
     reinterpret_cast<uint32_t*>(inf)[kInfoRowOff32 + rr] =
@@ -299,8 +306,8 @@ __device__ int wave_lower_bound(const BwdParams& p, int b, int lo, int hi, Pred 
 
 // One wave per (branch, key tile).
 template <bool kMeta>
-__global__ __launch_bounds__(kThreads) void bwd_ranges_kernel(const BwdParams p) {
-  const int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+__device__ __forceinline__ void block_ranges(const BwdParams& p, int wg) {
+  const int i = (wg * kThreads + threadIdx.x) >> 6;
   if (i >= 2 * p.kv_tiles_dkv) return;   // whole waves
   const int b = i / p.kv_tiles_dkv, t = i - b * p.kv_tiles_dkv;
   const int k0 = t * kKeysDkv, k1 = min(k0 + kKeysDkv, p.total_kv);
@@ -317,6 +324,18 @@ __global__ __launch_bounds__(kThreads) void bwd_ranges_kernel(const BwdParams p)
     p.ranges[2 * i] = blo;
     p.ranges[2 * i + 1] = bhi;
   }
+}
+
+// Row info and block ranges need nothing of each other: one launch, the short
+// latency-bound searches beside the HBM-bound blocks (a launch of their own
+// cost 3-5 us on the GPU).
+template <bool kMeta>
+__global__ __launch_bounds__(kThreads) void bwd_prep_kernel(const BwdParams p) {
+  const int wg = blockIdx.x;
+  if (wg < p.prep_wgs)
+    prep_block<kMeta>(p, wg);
+  else
+    block_ranges<kMeta>(p, wg - p.prep_wgs);
 }
 
 // ---------------------------------------------------------------------------
@@ -415,6 +434,37 @@ __device__ __forceinline__ void dkv_pair(const BwdParams& p, int r, int& t, int&
   }
 }
 
+// What dK/dV workgroup wg takes: share s of the row blocks of a (key tile t,
+// KV head) pair, first .. first + nb - 1 of its n0 full and n1 local blocks
+// (from block b0lo and b1lo on).  A pair of more than dkv_chunk blocks is cut
+// into nch equal shares, at most dkv_split; shorter pairs stay whole.
+// Share 0 of every pair comes first, then share 1, ...: the shares that do not
+// exist then spread evenly over the XCDs (workgroup i runs on XCD i % 8; pair
+// by pair, an even number of slots would leave them all on the same ones).
+struct DkvShare {
+  int t, kvh, s, nch, b0lo, b1lo, n0, n1, first, nb;
+};
+__device__ __forceinline__ int dkv_pieces(const BwdParams& p, int n) {
+  return max(1, min(p.dkv_split, (n + p.dkv_chunk - 1) / p.dkv_chunk));
+}
+__device__ __forceinline__ DkvShare dkv_share(const BwdParams& p, int wg) {
+  DkvShare d;
+  const int pairs = p.kv_tiles_dkv * p.hkv;
+  d.s = wg / pairs;
+  dkv_pair(p, wg - d.s * pairs, d.t, d.kvh);
+  const int nt = p.kv_tiles_dkv;
+  d.b0lo = p.ranges[2 * d.t];
+  d.b1lo = p.ranges[2 * (nt + d.t)];
+  d.n0 = max(p.ranges[2 * d.t + 1] - d.b0lo, 0);
+  d.n1 = max(p.ranges[2 * (nt + d.t) + 1] - d.b1lo, 0);
+  const int n = d.n0 + d.n1;
+  d.nch = dkv_pieces(p, n);
+  const int share = (n + d.nch - 1) / d.nch;
+  d.first = min(n, d.s * share);
+  d.nb = min(n - d.first, share);
+  return d;
+}
+
 // The bf16 dK / dV rows of one lane's key (lane half h) from its dK^T / dV^T
 // accumulators: element e of block d is d-row 32d + 8(e/4) + 4h + e%4.
 __device__ __forceinline__ void store_dkdv_rows(const BwdParams& p, int key, int kvh, int h,
@@ -445,6 +495,28 @@ __device__ __forceinline__ float4* part_unit(const BwdParams& p, int64_t wg, int
          lane;
 }
 
+// dQ workgroup wg takes piece s of row tile t (full ones first) for KV head
+// kvh: piece 0 of every full tile, then piece 1, ..., then the local tiles the
+// same way, KV head fastest.  (Like the dK/dV shares, pieces that do not exist
+// spread over the XCDs.)  dq_slot_wg is the inverse.
+__device__ __forceinline__ void dq_slot(const BwdParams& p, int wg, int& t, int& s, int& kvh) {
+  kvh = wg % p.hkv;
+  const int ts = wg / p.hkv, full_slots = p.items[0] * p.dq_maxc[0];
+  if (ts < full_slots) {
+    s = ts / p.items[0];
+    t = ts - s * p.items[0];
+  } else {
+    s = (ts - full_slots) / p.items[1];
+    t = p.items[0] + ts - full_slots - s * p.items[1];
+  }
+}
+__device__ __forceinline__ int64_t dq_slot_wg(const BwdParams& p, int t, int s, int kvh) {
+  const int64_t ts = t < p.items[0] ? static_cast<int64_t>(s) * p.items[0] + t
+                                    : static_cast<int64_t>(p.items[0]) * p.dq_maxc[0] +
+                                          static_cast<int64_t>(s) * p.items[1] + t - p.items[0];
+  return ts * p.hkv + kvh;
+}
+
 // Float4 unit u (= 4d + j: dQ^T block d elements 4j .. 4j+3) of (workgroup
 // wg, wave, lane) in the dQ piece partials.
 __device__ __forceinline__ float4* dq_part_unit(const BwdParams& p, int64_t wg, int wave, int u,
@@ -462,14 +534,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
   // stages, its source pointer) then stay scalar selects.
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
-  // Workgroup = (pair rank, split s): the rank gives the (key tile t, KV
-  // head) pair (dkv_pair); split s of dkv_split takes an equal share of the
-  // pair's row blocks (all of them without a split).
-  const int split = p.dkv_split;
-  const int pair = blockIdx.x / split;
-  const int s_idx = blockIdx.x - pair * split;
-  int t, kvh;
-  dkv_pair(p, pair, t, kvh);
+  const DkvShare sh = dkv_share(p, blockIdx.x);
+  if (sh.s >= sh.nch) return;
+  const int t = sh.t, kvh = sh.kvh;
   const int kw0 = t * kKeysDkv + 32 * wave;   // this wave's first key
   const int key = kw0 + n;                    // this lane's key (B column)
 
@@ -492,13 +559,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
 #pragma unroll
   for (int d = 0; d < 4; ++d) dkt[d] = dvt[d] = f32x16{};
 
-  const int nt = p.kv_tiles_dkv;
-  const int b0lo = p.ranges[2 * t], b0hi = p.ranges[2 * t + 1];
-  const int b1lo = p.ranges[2 * (nt + t)], b1hi = p.ranges[2 * (nt + t) + 1];
-  const int n0 = max(b0hi - b0lo, 0), n1 = max(b1hi - b1lo, 0);
-  const int chunk = (n0 + n1 + split - 1) / split;
-  const int first = min(n0 + n1, s_idx * chunk);
-  const int nb = min(n0 + n1 - first, chunk);   // this workgroup's blocks: first .. first+nb-1
+  const int b0lo = sh.b0lo, b1lo = sh.b1lo, n0 = sh.n0, first = sh.first;
+  const int nb = sh.nb;   // this workgroup's blocks: first .. first+nb-1
   auto block_of = [&](int i) -> int64_t {
     const int a = first + i;
     return a < n0 ? packed_block(p, 0, kvh, b0lo + a) : packed_block(p, 1, kvh, b1lo + a - n0);
@@ -624,11 +686,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
     }
   }
 
-  if (split == 1) {
+  if (sh.nch == 1) {
     store_dkdv_rows(p, key, kvh, h, dkt, dvt);
   } else {
-    // fp32 partials (zeros for a split with no blocks); bwd_dkdv_reduce_kernel
-    // sums the splits in order and stores the rows.
+    // fp32 partials (zeros for a share with no blocks); bwd_reduce_kernel sums
+    // the shares in order and stores the rows.
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
 #pragma unroll
@@ -643,8 +705,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
 }
 
 // ---------------------------------------------------------------------------
-// bwd_dkdv_wide_kernel: bwd_dkdv_kernel's (key tile, KV head) pairs with four
-// waves of 64 keys, one wave per SIMD, for grids that need no split.  Each
+// dkdv_wide (bwd_wide_kernel): bwd_dkdv_kernel's (key tile, KV head) pairs with
+// four waves of 64 keys, one wave per SIMD.  Each
 // LDS read of a block's Q or dO operand then feeds two MFMAs (both 32-key
 // halves of the wave), and the per-lane state (dK^T and dV^T in AGPRs; K,
 // the score and dP tiles and their bf16 packs in VGPRs) exceeds what a
@@ -657,27 +719,16 @@ constexpr int kDkvAuxGroups = SWATTN_BWD_DKDV_AUX_GROUPS;
 static_assert(SWATTN_BWD_DKDV_RING_OFF == kVTileBytes, "the V tile precedes the row ring");
 static_assert(4 * kDkvAuxGroups * 1024 <= 2 * 2 * kBlockBytes, "the inputs fit in ring slots 2-3");
 
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
-void bwd_dkdv_wide_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) char smem[kDkvWideLdsBytes];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+__device__ __forceinline__ void dkdv_wide(const BwdParams& p, char* smem, int wg, int wave) {
+  const int lane = count_below(~uint64_t{0});
   const int j = lane & 31, hh = lane >> 5;
-  // Workgroup = (pair rank, split s), as in bwd_dkdv_kernel: split s of
-  // dkv_split takes an equal share of the pair's row blocks in the loop's
-  // order (all of them without a split) and leaves fp32 partials.
-  const int split = p.dkv_split;
-  const int pair = blockIdx.x / split;
-  const int s_idx = blockIdx.x - pair * split;
-  int t, kvh;
-  dkv_pair(p, pair, t, kvh);
-  const int nt = p.kv_tiles_dkv;
-  const int b0lo = p.ranges[2 * t], b0hi = p.ranges[2 * t + 1];
-  const int b1lo = p.ranges[2 * (nt + t)], b1hi = p.ranges[2 * (nt + t) + 1];
-  const int n0 = max(b0hi - b0lo, 0), n1 = max(b1hi - b1lo, 0);
-  const int chunk = (n0 + n1 + split - 1) / split;
-  const int first = min(n0 + n1, s_idx * chunk);
-  const int nb = min(n0 + n1 - first, chunk);
+  // The pair's blocks run in the loop's order; a share of a cut pair leaves
+  // fp32 partials.
+  const DkvShare sh = dkv_share(p, wg);
+  if (sh.s >= sh.nch) return;   // uniform
+  const int t = sh.t, kvh = sh.kvh, b0lo = sh.b0lo, b1lo = sh.b1lo, n0 = sh.n0;
+  const int first = sh.first, nb = sh.nb;
+  const bool split = sh.nch > 1;
   const int pb0 = static_cast<int>(packed_block(p, 0, kvh, b0lo));
   const int pb1 = static_cast<int>(packed_block(p, 1, kvh, b1lo)) - n0;
   const int kw0 = t * kKeysDkv + 64 * wave;
@@ -745,10 +796,10 @@ void bwd_dkdv_wide_kernel(const BwdParams p) {
   const uint64_t vb64 = (static_cast<uint64_t>(vb_hi) << 32) | vb_lo;
   const float c = p.c, scale = p.scale;
   // This wave's split partials: the reduce's waves 2 wave and 2 wave + 1.
-  const char* part = split > 1 ? reinterpret_cast<const char*>(p.dkv_part) +
-                                     (static_cast<int64_t>(blockIdx.x) * kBwdWaves + 2 * wave) * kPartUnits * 1024
-                               : reinterpret_cast<const char*>(p.dk);
-  const i32x4 prsrc = make_rsrc(part, split > 1 ? 2 * kPartUnits * 1024 : 0);
+  const char* part = split ? reinterpret_cast<const char*>(p.dkv_part) +
+                                 (static_cast<int64_t>(wg) * kBwdWaves + 2 * wave) * kPartUnits * 1024
+                           : reinterpret_cast<const char*>(p.dk);
+  const i32x4 prsrc = make_rsrc(part, split ? 2 * kPartUnits * 1024 : 0);
   asm volatile(SWATTN_BWD_DKDV_ASM
                :
                : [qrsrc] "s"(qrsrc), [dorsrc] "s"(dorsrc), [irsrc] "s"(irsrc), [krsrc] "s"(krsrc),
@@ -758,7 +809,7 @@ void bwd_dkdv_wide_kernel(const BwdParams p) {
                  [pb1n] "s"(__builtin_amdgcn_readfirstlane(pb1 + n0)),
                  [pbf] "s"(__builtin_amdgcn_readfirstlane(pb0 + n0 - 1 - first)),
                  [pb1] "s"(__builtin_amdgcn_readfirstlane(pb1 + first)),
-                 [prsrc] "s"(prsrc), [split] "s"(__builtin_amdgcn_readfirstlane(split > 1 ? 1 : 0)),
+                 [prsrc] "s"(prsrc), [split] "s"(__builtin_amdgcn_readfirstlane(split ? 1 : 0)),
                  [kw0] "s"(__builtin_amdgcn_readfirstlane(kw0)),
                  [krow4] "s"(__builtin_amdgcn_readfirstlane(static_cast<int>(4 * krowbytes))),
                  [vl] "s"(__builtin_amdgcn_readfirstlane(lds0 + 64 * wave * kRowBytes)),
@@ -768,39 +819,56 @@ void bwd_dkdv_wide_kernel(const BwdParams p) {
                : SWATTN_BWD_DKDV_CLOBBERS);
 }
 
-// dK / dV of split pairs: one thread per (pair, wave, float4 unit, lane).
-// It sums that unit over the splits in split order (deterministic) and stores
-// its four bf16 values where the unsplit kernel's epilogue would.
+// dK / dV of cut pairs: a thread folds kUnits of (pair, wave, float4 unit,
+// lane).  It sums each unit over the shares in order (deterministic) and
+// stores its four bf16 values where the uncut kernel's epilogue would.
 static_assert(kPartUnits == 32 && kBwdWaves == 8, "the reduce's thread index splits 6 + 5 + 3 bits");
-__global__ __launch_bounds__(kThreads) void bwd_dkdv_reduce_kernel(const BwdParams p) {
-  const int64_t id = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  const int lane = static_cast<int>(id & 63);
-  const int u = static_cast<int>((id >> 6) & (kPartUnits - 1));
-  const int wave = static_cast<int>((id >> 11) & (kBwdWaves - 1));
-  const int pair = static_cast<int>(id >> 14);
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int sp = 0; sp < p.dkv_split; ++sp) {
-    const float4 a = *part_unit(p, static_cast<int64_t>(pair) * p.dkv_split + sp, wave, u, lane);
-    acc.x += a.x;
-    acc.y += a.y;
-    acc.z += a.z;
-    acc.w += a.w;
+constexpr int kDkvReduceWgs = kBwdWaves * kPartUnits * 64 / kThreads;   // per pair, at one unit each
+template <int kUnits>
+__device__ __forceinline__ void dkdv_reduce(const BwdParams& p, int wg) {
+  constexpr int kWgs = kDkvReduceWgs / kUnits;
+  const int pair = wg / kWgs;
+  const DkvShare sh = dkv_share(p, pair);
+  if (sh.nch <= 1) return;   // stored whole by its workgroup
+  const int kvh = sh.kvh;
+  const int64_t pairs = static_cast<int64_t>(p.kv_tiles_dkv) * p.hkv;
+  const int lane = threadIdx.x & 63;
+  // Unit i of the thread: id = (pair-relative workgroup, i, thread).
+  const int id0 = (wg - pair * kWgs) * kUnits * kThreads + threadIdx.x;
+  auto unit = [](int id) { return (id >> 6) & (kPartUnits - 1); };
+  auto wave_of = [](int id) { return id >> 11; };
+  float4 acc[kUnits];
+#pragma unroll
+  for (int i = 0; i < kUnits; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 2
+  for (int sp = 0; sp < sh.nch; ++sp) {
+#pragma unroll
+    for (int i = 0; i < kUnits; ++i) {
+      const int id = id0 + i * kThreads;
+      const float4 a = *part_unit(p, sp * pairs + pair, wave_of(id), unit(id), lane);
+      acc[i].x += a.x;
+      acc[i].y += a.y;
+      acc[i].z += a.z;
+      acc[i].w += a.w;
+    }
   }
-  int t, kvh;
-  dkv_pair(p, pair, t, kvh);
-  const int key = t * kKeysDkv + 32 * wave + (lane & 31);
-  if (key >= p.total_kv) return;
-  // Unit 4d + j (+16 for dV): elements 4j .. 4j+3 of block d, i.e. d-rows
-  // 32d + 8j + 4h .. +3 of the key (lane half h).
-  const bool is_v = u >= 16;
-  const int d = (u & 15) >> 2, j = u & 3;
-  const float sc = is_v ? 1.0f : p.scale;
-  uint2 w;
-  w.x = pack_bf16x2(acc.x * sc, acc.y * sc);
-  w.y = pack_bf16x2(acc.z * sc, acc.w * sc);
-  uint16_t* dst = is_v ? p.dv : p.dk;
-  *reinterpret_cast<uint2*>(dst + (static_cast<int64_t>(key) * p.hkv + kvh) * kD + 4 * (lane >> 5) +
-                            32 * d + 8 * j) = w;
+#pragma unroll
+  for (int i = 0; i < kUnits; ++i) {
+    const int u = unit(id0 + i * kThreads);
+    const int key = sh.t * kKeysDkv + 32 * wave_of(id0 + i * kThreads) + (lane & 31);
+    if (key >= p.total_kv) continue;
+    // Unit 4d + j (+16 for dV): elements 4j .. 4j+3 of block d, i.e. d-rows
+    // 32d + 8j + 4h .. +3 of the key (lane half h).
+    const bool is_v = u >= 16;
+    const int d = (u & 15) >> 2, j = u & 3;
+    const float sc = is_v ? 1.0f : p.scale;
+    uint2 w;
+    w.x = pack_bf16x2(acc[i].x * sc, acc[i].y * sc);
+    w.y = pack_bf16x2(acc[i].z * sc, acc[i].w * sc);
+    uint16_t* dst = is_v ? p.dv : p.dk;
+    *reinterpret_cast<uint2*>(dst + (static_cast<int64_t>(key) * p.hkv + kvh) * kD + 4 * (lane >> 5) +
+                              32 * d + 8 * j) = w;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -854,13 +922,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
   const int n = lane & 31, h = lane >> 5;
   // Workgroup = ((row tile t, piece slot s), KV head), KV head fastest; a
   // row tile of branch b has dq_maxc[b] consecutive slots.
-  const int kvh = blockIdx.x % p.hkv;
-  const int ts = blockIdx.x / p.hkv;
-  const int full_slots = p.items[0] * p.dq_maxc[0];
-  const int t = ts < full_slots ? ts / p.dq_maxc[0]
-                                : p.items[0] + (ts - full_slots) / p.dq_maxc[1];
-  const int s_idx = ts < full_slots ? ts - t * p.dq_maxc[0]
-                                    : ts - full_slots - (t - p.items[0]) * p.dq_maxc[1];
+  int t, s_idx, kvh;
+  dq_slot(p, blockIdx.x, t, s_idx, kvh);
   const int b = t < p.items[0] ? 0 : 1;
   // Latest positions first in each branch (longest rows first).
   const int item = b == 0 ? p.items[0] - 1 - t : p.items[0] + p.items[1] - 1 - t;
@@ -1035,7 +1098,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
 
   const int G = p.group;
   if (piece) {
-    // fp32 partials (zeros for a piece with no tiles); bwd_dq_reduce_kernel
+    // fp32 partials (zeros for a piece with no tiles); bwd_reduce_kernel
     // sums the pieces in order and stores the rows.
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
@@ -1065,7 +1128,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
 }
 
 // ---------------------------------------------------------------------------
-// bwd_dq_wide_kernel: bwd_dq_kernel's work items with four waves of 64 rows,
+// dq_wide (bwd_wide_kernel): bwd_dq_kernel's work items with four waves of 64 rows,
 // one wave per SIMD.  Each K / V operand read from LDS then feeds two MFMAs
 // (both 32-row blocks of the wave), and the per-lane state (dQ^T, Q^T and
 // dO^T in AGPRs; two score tiles, the dP tile and the operand staging in
@@ -1086,21 +1149,13 @@ __device__ __forceinline__ int dq_aux_offset(int wave) {
 }
 static_assert(2 * kDqAuxGroups * 1024 <= kTileBytes, "two waves' inputs fit in a ring slot");
 
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
-void bwd_dq_wide_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) char smem[kDqWideLdsBytes];
-  __shared__ int s_range[8];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+__device__ __forceinline__ void dq_wide(const BwdParams& p, char* smem, int* s_range, int wg,
+                                        int wave) {
+  const int lane = count_below(~uint64_t{0});
   const int n = lane & 31, h = lane >> 5;
   // Workgroup = ((row tile t, piece slot s), KV head) as in bwd_dq_kernel.
-  const int kvh = blockIdx.x % p.hkv;
-  const int ts = blockIdx.x / p.hkv;
-  const int full_slots = p.items[0] * p.dq_maxc[0];
-  const int t = ts < full_slots ? ts / p.dq_maxc[0]
-                                : p.items[0] + (ts - full_slots) / p.dq_maxc[1];
-  const int s_idx = ts < full_slots ? ts - t * p.dq_maxc[0]
-                                    : ts - full_slots - (t - p.items[0]) * p.dq_maxc[1];
+  int t, s_idx, kvh;
+  dq_slot(p, wg, t, s_idx, kvh);
   const int b = t < p.items[0] ? 0 : 1;
   const int item = b == 0 ? p.items[0] - 1 - t : p.items[0] + p.items[1] - 1 - t;
 
@@ -1142,6 +1197,8 @@ void bwd_dq_wide_kernel(const BwdParams p) {
     g_s = min(g_s, s_range[i]);
     g_e = max(g_e, s_range[4 + i]);
   }
+  g_s = __builtin_amdgcn_readfirstlane(g_s);   // scalar, so that the return below is a scalar branch
+  g_e = __builtin_amdgcn_readfirstlane(g_e);
   const int t_all0 = g_e > g_s ? g_s / kBN : 0;
   const int t_all1 = g_e > g_s ? (g_e + kBN - 1) / kBN : 0;
   int t_begin = t_all0, t_end = t_all1;
@@ -1150,7 +1207,7 @@ void bwd_dq_wide_kernel(const BwdParams p) {
     const int len = t_all1 - t_all0;
     const int nch = max(1, min(p.dq_maxc[b], (len + p.dq_chunk - 1) / p.dq_chunk));
     if (s_idx >= nch) return;
-    if (s_idx == 0 && tid == 0) p.dq_nch[t * p.hkv + kvh] = nch;
+    if (s_idx == 0 && wave == 0 && lane == 0) p.dq_nch[t * p.hkv + kvh] = nch;
     piece = nch > 1;
     const int plen = (len + nch - 1) / nch;
     t_begin = t_all0 + min(len, s_idx * plen);
@@ -1240,7 +1297,7 @@ void bwd_dq_wide_kernel(const BwdParams p) {
   const i32x4 dqrsrc = make_rsrc(p.dq, qbytes);
   // This wave's pieces partials: units of row blocks 2 wave and 2 wave + 1.
   const char* part = reinterpret_cast<const char*>(p.dq_part) +
-                     (static_cast<int64_t>(blockIdx.x) * kBwdWaves + 2 * wave) * kDqPartUnits * 1024;
+                     (static_cast<int64_t>(wg) * kBwdWaves + 2 * wave) * kDqPartUnits * 1024;
   const i32x4 prsrc = make_rsrc(piece ? part : reinterpret_cast<const char*>(p.dq), piece ? 2 * kDqPartUnits * 1024 : 0);
   const uint32_t kb_lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(kbase));
   const uint32_t kb_hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(kbase >> 32));
@@ -1266,70 +1323,117 @@ void bwd_dq_wide_kernel(const BwdParams p) {
                : SWATTN_BWD_DQ_CLOBBERS);
 }
 
-// dQ of row tiles cut into pieces: one thread per (row tile and KV head,
-// wave, float4 unit, lane); row tiles left whole were stored by the dQ
-// kernel.  It sums that unit over the pieces in piece order
-// (deterministic) and stores its four bf16 values where a whole row tile
-// would: the lane's row of the tile, d-rows 32d + 8j + 4h .. +3.
+// Both products in one grid, dK/dV's workgroups first: dQ's fill the CUs that
+// dK/dV's last (longest) workgroups leave idle, and a small grid runs both at
+// once.  With that, pairs need cutting less often: at B2 S4096 Hq32/Hkv8 W1024
+// none is (307 us + 31 us of reduce + 225 us of dQ -> 524 us for both); B1
+// S1024 Hq8/Hkv2: 20.6 + 18.7 -> 22.6 us; B1 S16384 Hq32/Hkv8 1 % less.
+constexpr int kWideLdsBytes = kDkvWideLdsBytes > kDqWideLdsBytes ? kDkvWideLdsBytes : kDqWideLdsBytes;
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void bwd_wide_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) char smem[kWideLdsBytes];
+  __shared__ int s_range[8];
+  const int wg = blockIdx.x;
+  // The wave as a scalar, the lane counted where it is used: a thread index
+  // in a register would be kept alive across a branch's loop, in scratch.
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wg < p.dkv_wgs)
+    dkdv_wide(p, smem, wg, wave);
+  else
+    dq_wide(p, smem, s_range, wg - p.dkv_wgs, wave);
+}
+
+// dQ of row tiles cut into pieces: a thread folds kUnits of (row tile and KV
+// head, wave, float4 unit, lane); row tiles left whole were stored by the dQ
+// kernel.  It sums each unit over the pieces in piece order (deterministic) and
+// stores its four bf16 values where a whole row tile would: the lane's row of
+// the tile, d-rows 32d + 8j + 4h .. +3.
 static_assert(kDqPartUnits == 16 && kBwdWaves == 8, "the reduce's thread index splits 6 + 4 + 3 bits");
-__global__ __launch_bounds__(kThreads) void bwd_dq_reduce_kernel(const BwdParams p) {
-  const int64_t id = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  const int lane = static_cast<int>(id & 63);
-  const int u = static_cast<int>((id >> 6) & (kDqPartUnits - 1));
-  const int wave = static_cast<int>((id >> 10) & (kBwdWaves - 1));
-  const int tk = static_cast<int>(id >> 13);   // (row tile t, KV head), KV head fastest
+constexpr int kDqReduceWgs = kBwdWaves * kDqPartUnits * 64 / kThreads;   // per tile, at one unit each
+template <int kUnits>
+__device__ __forceinline__ void dq_reduce(const BwdParams& p, int wg) {
+  constexpr int kWgs = kDqReduceWgs / kUnits;
+  const int tk = wg / kWgs;   // (row tile t, KV head), KV head fastest
   const int kvh = tk % p.hkv, t = tk / p.hkv;
   const int nch = p.dq_nch[tk];
   if (nch <= 1) return;
-  // The row tile's first workgroup slot (slots are ordered as the dQ grid).
-  const int64_t slot0 = t < p.items[0]
-                            ? static_cast<int64_t>(t) * p.dq_maxc[0]
-                            : static_cast<int64_t>(p.items[0]) * p.dq_maxc[0] +
-                                  static_cast<int64_t>(t - p.items[0]) * p.dq_maxc[1];
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int lane = threadIdx.x & 63;
+  const int id0 = (wg - tk * kWgs) * kUnits * kThreads + threadIdx.x;
+  auto unit = [](int id) { return (id >> 6) & (kDqPartUnits - 1); };
+  auto wave_of = [](int id) { return id >> 10; };
+  float4 acc[kUnits];
+#pragma unroll
+  for (int i = 0; i < kUnits; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 2
   for (int sp = 0; sp < nch; ++sp) {
-    const int64_t wg = (slot0 + sp) * p.hkv + kvh;
-    const float4 a = *dq_part_unit(p, wg, wave, u, lane);
-    acc.x += a.x;
-    acc.y += a.y;
-    acc.z += a.z;
-    acc.w += a.w;
+    const int64_t piece = dq_slot_wg(p, t, sp, kvh);
+#pragma unroll
+    for (int i = 0; i < kUnits; ++i) {
+      const int id = id0 + i * kThreads;
+      const float4 a = *dq_part_unit(p, piece, wave_of(id), unit(id), lane);
+      acc[i].x += a.x;
+      acc[i].y += a.y;
+      acc[i].z += a.z;
+      acc[i].w += a.w;
+    }
   }
   const int b = t < p.items[0] ? 0 : 1;
   const int item = b == 0 ? p.items[0] - 1 - t : p.items[0] + p.items[1] - 1 - t;
-  const int blk = item * (kRowsPerItem / kBRows) + wave;
-  const int r = blk * kBRows + (lane & 31);
-  if (blk >= p.blocks[b] || r >= p.nrows[b]) return;
   const int G = p.group;
-  const int q_slot = r / G;
-  const int pos = p.idx[b][q_slot];
-  if (!pos_ok(p, pos)) return;
-  const int qh = kvh * G + (r - q_slot * G);
-  const int d = u >> 2, j = u & 3;
-  uint2 w;
-  w.x = pack_bf16x2(acc.x * p.scale, acc.y * p.scale);
-  w.y = pack_bf16x2(acc.z * p.scale, acc.w * p.scale);
-  *reinterpret_cast<uint2*>(p.dq + (static_cast<int64_t>(pos) * p.hq + qh) * kD +
-                            4 * (lane >> 5) + 32 * d + 8 * j) = w;
+#pragma unroll
+  for (int i = 0; i < kUnits; ++i) {
+    const int u = unit(id0 + i * kThreads);
+    const int blk = item * (kRowsPerItem / kBRows) + wave_of(id0 + i * kThreads);
+    const int r = blk * kBRows + (lane & 31);
+    if (blk >= p.blocks[b] || r >= p.nrows[b]) continue;
+    const int q_slot = r / G;
+    const int pos = p.idx[b][q_slot];
+    if (!pos_ok(p, pos)) continue;
+    const int qh = kvh * G + (r - q_slot * G);
+    const int d = u >> 2, j = u & 3;
+    uint2 w;
+    w.x = pack_bf16x2(acc[i].x * p.scale, acc[i].y * p.scale);
+    w.y = pack_bf16x2(acc[i].z * p.scale, acc[i].w * p.scale);
+    *reinterpret_cast<uint2*>(p.dq + (static_cast<int64_t>(pos) * p.hq + qh) * kD +
+                              4 * (lane >> 5) + 32 * d + 8 * j) = w;
+  }
+}
+
+// Both reduces in one launch: workgroups below dkv_wgs fold dK/dV partials, the
+// rest dQ's.  With kUnits = 4 a thread has four units' loads in flight and the
+// grid a quarter of the waves (at 256 pairs, launching a wave per unit took
+// 11 us even where no pair is cut); small grids need every wave they can get
+// (B1 S1024 Hq8/Hkv2: 7.7 us with one unit, 11.5 with four).
+template <int kUnits>
+__global__ __launch_bounds__(kThreads) void bwd_reduce_kernel(const BwdParams p) {
+  const int wg = blockIdx.x;
+  if (wg < p.dkv_wgs)
+    dkdv_reduce<kUnits>(p, wg);
+  else
+    dq_reduce<kUnits>(p, wg - p.dkv_wgs);
 }
 
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
+// Reduce grids (in workgroups of one unit per thread) from this size on take
+// four units per thread: 16 workgroups per CU.
+constexpr int64_t kReduceWide = 4096;
+
 struct BwdLayout {
-  int64_t blocks[2], items[2], total_blocks, kv_tiles_dkv, dkv_split, dq_chunk, dq_maxc[2];
+  int64_t blocks[2], items[2], total_blocks, kv_tiles_dkv, dkv_split, dkv_chunk, dq_chunk, dq_maxc[2];
   size_t off_info, off_zero, off_ranges, off_part, off_dq_nch, off_dq_part, bytes;
 };
 
 inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
-// bwd_dq_wide_kernel addresses Q, dO, dq and the item's K / V bytes with
+// dq_wide addresses Q, dO, dq and the item's K / V bytes with
 // 32-bit buffer offsets (and drops out-of-range ones): both must stay below
 // 2^31 bytes.  SWATTN_DQ_KERNEL=narrow / wide picks a kernel for tests and
 // comparisons.
-// bwd_dkdv_wide_kernel gathers rows by 32-bit offsets into Q / dO and reads
+// dkdv_wide gathers rows by 32-bit offsets into Q / dO and reads
 // K, V, dK, dV and the row info through 32-bit buffer ranges (all below
-// 2^31 bytes).  It runs split or unsplit, as the layout decides;
+// 2^31 bytes).
 // SWATTN_DKDV_KERNEL=narrow picks the eight-wave kernel (tests and
 // comparisons).
 inline bool use_dkdv_wide(int64_t total_q, int64_t total_kv, int32_t heads_q, int32_t heads_kv,
@@ -1360,9 +1464,10 @@ inline BwdLayout bwd_layout(int64_t seq_kv, int64_t total_kv, int32_t heads_kv, 
   }
   L.total_blocks = static_cast<int64_t>(heads_kv) * (L.blocks[0] + L.blocks[1]);
   L.kv_tiles_dkv = ceil_div(total_kv, kKeysDkv);
-  // Fewer (key tile, KV head) pairs than two rounds of workgroups: each pair
-  // is split over its row blocks, so that the longest pair (the first key
-  // tile sees every full row) no longer sets the kernel's length.
+  // Fewer (key tile, KV head) pairs than two rounds of workgroups: room to cut
+  // each pair over its row blocks, so that the longest pair (the first key
+  // tile sees every full row) does not set the grid's length (dkv_chunk below
+  // says which pairs are cut).
   const int64_t pairs = L.kv_tiles_dkv * heads_kv;
   L.dkv_split = pairs >= kDkvTargetWgs ? 1
                 : std::min<int64_t>(kDkvMaxSplit, ceil_div(kDkvTargetWgs, pairs));
@@ -1410,6 +1515,21 @@ inline BwdLayout bwd_layout(int64_t seq_kv, int64_t total_kv, int32_t heads_kv, 
     o += static_cast<size_t>(heads_kv * slots) * kDqPartBytesPerWg;
   }
   L.bytes = o;
+
+  // Within that room, the row blocks a dK/dV workgroup may take: as many as
+  // the grid has time per CU.  Both products run in one grid
+  // (bwd_wide_kernel), so a pair is too long only against all of it; cutting
+  // finer writes and reads back 256 KiB of partials more per workgroup.  (Times
+  // in tenths of a us: a row block 16, a dQ key tile 22, starting and ending a
+  // workgroup 150.  Shares of 1/2, 3/4 and 1 of the time per CU, forward and
+  // backward on the GPU: B1 S2048 Hq32/Hkv8 W512 192, 173 and 159 us; B1
+  // S16384 Hq4/Hkv1 W1024 477, 464 and 456; B2 S4096 Hq32/Hkv8 774, 732, 732;
+  // 5/4 of it would leave the last of two rounds half empty.)
+  const int64_t full_kt = ceil_div(seq_kv, kKeysDkv);
+  const int64_t local_kt = std::min<int64_t>(full_kt, ceil_div(window, kKeysDkv) + 1);
+  const int64_t dkv = heads_kv * (L.blocks[0] * (full_kt + 1) / 2 + L.blocks[1] * local_kt);
+  const int64_t per_cu = (16 * dkv + 150 * pairs + 22 * est + 150 * q_items) / kDqSlots;
+  L.dkv_chunk = std::min<int64_t>(INT32_MAX / 2, std::max<int64_t>(kDkvMinBlocks, (per_cu - 150) / 16));
   return L;
 }
 
@@ -1482,10 +1602,9 @@ extern "C" int swattn_prefill_bwd(const void* q, const void* k, const void* v, c
     return SWATTN_EWORKSPACE;
   }
   if (!aligned256(workspace)) return invalid("swattn_prefill_bwd: workspace must be 256-byte aligned");
-  if (L.kv_tiles_dkv * heads_kv * L.dkv_split > INT32_MAX ||
-      (L.items[0] * L.dq_maxc[0] + L.items[1] * L.dq_maxc[1]) * heads_kv > INT32_MAX ||
-      (L.dq_chunk > 0 &&
-       (L.items[0] + L.items[1]) * heads_kv * kBwdWaves * kDqPartUnits * 64 / kThreads > INT32_MAX))
+  if (L.kv_tiles_dkv * heads_kv * L.dkv_split +
+              (L.items[0] * L.dq_maxc[0] + L.items[1] * L.dq_maxc[1]) * heads_kv > INT32_MAX ||
+      (L.dq_chunk > 0 && (L.items[0] + L.items[1]) * heads_kv * kDqReduceWgs > INT32_MAX / 2))
     return invalid("swattn_prefill_bwd: grid too large");
 
   char* ws = static_cast<char*>(workspace);
@@ -1522,6 +1641,7 @@ extern "C" int swattn_prefill_bwd(const void* q, const void* k, const void* v, c
   p.total_kv = static_cast<int32_t>(total_kv);
   p.kv_tiles_dkv = static_cast<int32_t>(L.kv_tiles_dkv);
   p.dkv_split = static_cast<int32_t>(L.dkv_split);
+  p.dkv_chunk = static_cast<int32_t>(L.dkv_chunk);
   // Several sequences that each hold whole 256-key tiles: interleave them.
   p.dkv_batches = (batch > 1 && seq_kv % kKeysDkv == 0) ? batch : 1;
   p.dkv_part = reinterpret_cast<float*>(ws + L.off_part);
@@ -1538,44 +1658,41 @@ extern "C" int swattn_prefill_bwd(const void* q, const void* k, const void* v, c
   p.scale = scale_log2 * 0.69314718055994531f;   // sm_scale = c * ln 2
 
   const hipStream_t st = as_stream(stream);
-  const uint32_t rgrid = static_cast<uint32_t>(ceil_div(2 * L.kv_tiles_dkv, kThreads / 64));
+  const int64_t prep_wgs = (L.blocks[0] + L.blocks[1]) * heads_kv;
+  const int64_t range_wgs = ceil_div(2 * L.kv_tiles_dkv, kThreads / 64);
+  if (prep_wgs + range_wgs > INT32_MAX) return invalid("swattn_prefill_bwd: grid too large");
+  p.prep_wgs = static_cast<int32_t>(prep_wgs);
+  const dim3 gp(static_cast<uint32_t>(prep_wgs + range_wgs));
   if (meta)
-    hipLaunchKernelGGL(bwd_ranges_kernel<true>, dim3(rgrid), dim3(kThreads), 0, st, p);
+    hipLaunchKernelGGL(bwd_prep_kernel<true>, gp, dim3(kThreads), 0, st, p);
   else
-    hipLaunchKernelGGL(bwd_ranges_kernel<false>, dim3(rgrid), dim3(kThreads), 0, st, p);
-  const int64_t nblk = L.blocks[0] + L.blocks[1];
-  if (nblk > 0) {
-    if (meta)
-      hipLaunchKernelGGL(bwd_prep_kernel<true>, dim3(static_cast<uint32_t>(nblk), heads_kv),
-                         dim3(kThreads), 0, st, p);
-    else
-      hipLaunchKernelGGL(bwd_prep_kernel<false>, dim3(static_cast<uint32_t>(nblk), heads_kv),
-                         dim3(kThreads), 0, st, p);
-  }
+    hipLaunchKernelGGL(bwd_prep_kernel<false>, gp, dim3(kThreads), 0, st, p);
   const int64_t pairs = L.kv_tiles_dkv * heads_kv;
-  const bool dkdv_wide = use_dkdv_wide(total_q, total_kv, heads_q, heads_kv, L.total_blocks);
-  if (dkdv_wide)
-    hipLaunchKernelGGL(bwd_dkdv_wide_kernel, dim3(static_cast<uint32_t>(pairs * L.dkv_split)), dim3(256), 0,
-                       st, p);
-  else
-    hipLaunchKernelGGL(bwd_dkdv_kernel, dim3(static_cast<uint32_t>(pairs * L.dkv_split)),
-                       dim3(kBwdThreads), 0, st, p);
-  if (L.dkv_split > 1)
-    hipLaunchKernelGGL(bwd_dkdv_reduce_kernel,
-                       dim3(static_cast<uint32_t>(pairs * kBwdWaves * kPartUnits * 64 / kThreads)),
-                       dim3(kThreads), 0, st, p);
   const int64_t q_items = (L.items[0] + L.items[1]) * heads_kv;
-  if (q_items > 0) {
-    const int64_t dq_wgs = (L.items[0] * L.dq_maxc[0] + L.items[1] * L.dq_maxc[1]) * heads_kv;
-    if (use_dq_wide(total_q, total_kv, heads_q, heads_kv))
-      hipLaunchKernelGGL(bwd_dq_wide_kernel, dim3(static_cast<uint32_t>(dq_wgs)), dim3(256), 0, st, p);
+  const int64_t dkv_wgs = pairs * L.dkv_split;
+  const int64_t dq_wgs = (L.items[0] * L.dq_maxc[0] + L.items[1] * L.dq_maxc[1]) * heads_kv;
+  const bool dkdv_wide = use_dkdv_wide(total_q, total_kv, heads_q, heads_kv, L.total_blocks);
+  const bool dq_wide = use_dq_wide(total_q, total_kv, heads_q, heads_kv);
+  if (!dkdv_wide)
+    hipLaunchKernelGGL(bwd_dkdv_kernel, dim3(static_cast<uint32_t>(dkv_wgs)), dim3(kBwdThreads), 0,
+                       st, p);
+  if (!dq_wide && q_items > 0)
+    hipLaunchKernelGGL(bwd_dq_kernel, dim3(static_cast<uint32_t>(dq_wgs)), dim3(kBwdThreads), 0, st, p);
+  p.dkv_wgs = dkdv_wide ? static_cast<int32_t>(dkv_wgs) : 0;
+  const int64_t wide_wgs = p.dkv_wgs + (dq_wide ? dq_wgs : 0);
+  if (wide_wgs > 0)
+    hipLaunchKernelGGL(bwd_wide_kernel, dim3(static_cast<uint32_t>(wide_wgs)), dim3(256), 0, st, p);
+  // Partials of cut pairs and row tiles.
+  const int64_t dkv_red = L.dkv_split > 1 ? pairs * kDkvReduceWgs : 0;
+  const int64_t dq_red = L.dq_chunk > 0 ? q_items * kDqReduceWgs : 0;
+  const int units = dkv_red + dq_red >= kReduceWide ? 4 : 1;
+  p.dkv_wgs = static_cast<int32_t>(dkv_red / units);
+  const dim3 gr(static_cast<uint32_t>((dkv_red + dq_red) / units));
+  if (gr.x > 0) {
+    if (units == 4)
+      hipLaunchKernelGGL(bwd_reduce_kernel<4>, gr, dim3(kThreads), 0, st, p);
     else
-      hipLaunchKernelGGL(bwd_dq_kernel, dim3(static_cast<uint32_t>(dq_wgs)), dim3(kBwdThreads), 0,
-                         st, p);
-    if (L.dq_chunk > 0)
-      hipLaunchKernelGGL(bwd_dq_reduce_kernel,
-                         dim3(static_cast<uint32_t>(q_items * kBwdWaves * kDqPartUnits * 64 / kThreads)),
-                         dim3(kThreads), 0, st, p);
+      hipLaunchKernelGGL(bwd_reduce_kernel<1>, gr, dim3(kThreads), 0, st, p);
   }
   return launch_status("swattn_prefill_bwd");
 }
