@@ -469,13 +469,19 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads),
   const int rl = lane & 31, hh = lane >> 5;
 
   // ---- work item -> (branch, tile, chunk slot, kv head) ----------------------
-  // Full tiles come first, each as maxc chunk slots in a row; KV head fastest.
+  // Full tiles come first; KV head fastest.  Split: chunk slot 0 of every full
+  // tile, then slot 1, ..., so that the slots past an item's last chunk spread
+  // over the XCDs (workgroup i runs on XCD i % 8; tile by tile, an even number
+  // of slots on few KV heads leaves them all on the same ones: B1 S8192
+  // Hq8/Hkv2 W1024 took 117 us that way, 86 this way; S1500 Hq32/Hkv8 W300
+  // 43.0 and 34.8; S16384 Hq4/Hkv1, five slots, 123 either way).
   const int item = blockIdx.x;
   const int kvh = item % p.hkv;
   const int tq = item / p.hkv;
   const int full_slots = kSplit ? p.tiles[0] * p.maxc : p.tiles[0];
-  const int t = !kSplit ? tq : tq < full_slots ? tq / p.maxc : p.tiles[0] + (tq - full_slots);
-  const int cslot = kSplit && tq < full_slots ? tq - t * p.maxc : 0;
+  const int cslot = kSplit && tq < full_slots ? tq / p.tiles[0] : 0;
+  const int t = !kSplit ? tq
+                : tq < full_slots ? tq - cslot * p.tiles[0] : p.tiles[0] + (tq - full_slots);
   const int branch = t < p.tiles[0] ? 0 : 1;
   // Both branches run their last tile (latest positions) first: full tiles
   // are then ordered by falling causal length, and the local tiles that end
