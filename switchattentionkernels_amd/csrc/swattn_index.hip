@@ -19,9 +19,10 @@ namespace {
 // ---------------------------------------------------------------------------
 // Compaction (V:306-322).
 //
-// A block of 16 waves owns 16384 consecutive mask bytes; wave w owns 16 groups
-// of 64 bytes.  Lane l of group e reads byte base + 64e + l, so each group is
-// one coalesced 64-byte read and one 64-bit ballot.  popcount(ballot) gives the
+// A block of 16 waves owns 4096 or (long masks) 16384 consecutive mask bytes;
+// wave w owns 4 or 16 groups of 64 bytes.  Lane l of group e reads byte base +
+// 64e + l, so each group is one coalesced 64-byte read and one 64-bit ballot.
+// popcount(ballot) gives the
 // group's full count and mbcnt(ballot) a lane's rank inside the group; the
 // ballots stay in scalar registers between the counting pass and the write
 // pass, so the mask is read once per kernel.  Full position i lands at
@@ -37,33 +38,155 @@ constexpr int kCompactChunk = kCompactThreads * kCompactGroups;  // 16384 bytes 
 // What decides "full" for position i: a byte mask, or router logits above a
 // threshold (compared in fp32; bf16 and fp16 convert exactly, NaN is never
 // above the threshold).
+// count16: how many of the 16 bytes' values are full (kPer of them).
 struct MaskSource {
+  static constexpr int kPer = 16;
   const uint8_t* p;
   __device__ __forceinline__ bool operator()(int64_t i) const { return p[i] != 0; }
+  __device__ __forceinline__ int count16(const uint4& v) const {
+    auto nonzero = [](uint32_t x) {   // bytes of x that are not 0
+      return __builtin_popcount((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u);
+    };
+    return nonzero(v.x) + nonzero(v.y) + nonzero(v.z) + nonzero(v.w);
+  }
 };
 struct F32LogitSource {
+  static constexpr int kPer = 4;
   const float* p;
   float thr;
   __device__ __forceinline__ bool operator()(int64_t i) const { return p[i] > thr; }
+  __device__ __forceinline__ int count16(const uint4& v) const {
+    return (__uint_as_float(v.x) > thr) + (__uint_as_float(v.y) > thr) +
+           (__uint_as_float(v.z) > thr) + (__uint_as_float(v.w) > thr);
+  }
 };
 struct BF16LogitSource {
+  static constexpr int kPer = 8;
   const uint16_t* p;
   float thr;
   __device__ __forceinline__ bool operator()(int64_t i) const {
     return __uint_as_float(static_cast<uint32_t>(p[i]) << 16) > thr;
   }
+  __device__ __forceinline__ int count16(const uint4& v) const {
+    auto both = [this](uint32_t x) {
+      return (__uint_as_float(x << 16) > thr) + (__uint_as_float(x & 0xffff0000u) > thr);
+    };
+    return both(v.x) + both(v.y) + both(v.z) + both(v.w);
+  }
 };
 struct F16LogitSource {
+  static constexpr int kPer = 8;
   const _Float16* p;
   float thr;
   __device__ __forceinline__ bool operator()(int64_t i) const {
     return static_cast<float>(p[i]) > thr;
   }
+  __device__ __forceinline__ int count16(const uint4& v) const {
+    auto both = [this](uint32_t x) {
+      const auto h = __builtin_bit_cast(__attribute__((ext_vector_type(2))) _Float16, x);
+      return (static_cast<float>(h.x) > thr) + (static_cast<float>(h.y) > thr);
+    };
+    return both(v.x) + both(v.y) + both(v.z) + both(v.w);
+  }
 };
 
+// Position of lane `lane` of group e of wave `wave`, kGroups groups per wave.
+template <int kGroups>
 __device__ __forceinline__ int64_t compact_elem(int wave, int e, int lane) {
-  return static_cast<int64_t>(blockIdx.x) * kCompactChunk +
-         static_cast<int64_t>(wave) * (64 * kCompactGroups) + 64 * e + lane;
+  return (static_cast<int64_t>(blockIdx.x) * kCompactWaves + wave) * (64 * kGroups) + 64 * e + lane;
+}
+
+// The write pass of a block: its ballots, the full positions before the wave
+// (all of the mask's before the block included) and in all of the mask.
+template <int kGroups>
+__device__ __forceinline__ void compact_write(const uint64_t (&bal)[kGroups], int64_t full_before,
+                                              int64_t nf, int64_t n, int32_t* __restrict__ indices) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int e = 0; e < kGroups; ++e) {
+    const int64_t i = compact_elem<kGroups>(wave, e, lane);
+    const uint64_t b = bal[e];
+    const int64_t fb = full_before + count_below(b);
+    if (i < n) {
+      if ((b >> lane) & 1ull)
+        indices[fb] = static_cast<int32_t>(i);
+      else
+        indices[nf + (i - fb)] = static_cast<int32_t>(i);
+    }
+    full_before += __builtin_popcountll(b);
+  }
+}
+
+// One launch, for masks that every block can afford to read whole: a block
+// writes 4096 positions and counts the full ones of all the mask, those before
+// its own apart, from L2 (16 bytes per lane and load where the mask is
+// 16-byte aligned).  Latency-bound: against one block for all 16384 positions
+// this spreads the loads and the stores over CUs, and against a counting
+// kernel first it saves that launch.  Back to back, byte mask: 1024 positions
+// 4.6 -> 2.8 us, 16384 5.9 -> 4.1, 65536 9.6 (two kernels) -> 4.6, 262144 10.1 ->
+// 6.6; fp32 logits: 16384 6.0 -> 4.5, 65536 10.0 -> 6.2.
+constexpr int kWholeGroups = 4;
+constexpr int kWholeChunk = kCompactThreads * kWholeGroups;   // 4096 positions per block
+constexpr int64_t kWholeBytes = 256 << 10;   // a block reads at most this much (10 us, as two kernels)
+constexpr int64_t kWholeUnaligned = 64 << 10;   // positions, read one by one (8 us; 131072: 12)
+template <typename Src, bool kVec>
+__global__ __launch_bounds__(kCompactThreads) void compact_whole_kernel(
+    const Src src, int64_t n, int32_t* __restrict__ indices, int32_t* __restrict__ counts) {
+  __shared__ int s_own[kCompactWaves], s_before[kCompactWaves], s_all[kCompactWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint64_t bal[kWholeGroups];
+  int own = 0;
+#pragma unroll
+  for (int e = 0; e < kWholeGroups; ++e) {
+    const int64_t i = compact_elem<kWholeGroups>(wave, e, lane);
+    const bool f = i < n && src(i);
+    bal[e] = wave_ballot(f);
+    own += __builtin_popcountll(bal[e]);
+  }
+  int before = 0, all = 0;
+  if (gridDim.x > 1) {
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kWholeChunk;
+    int64_t done = 0;
+    if constexpr (kVec) {   // kPer divides the chunk: a load is before it or not
+      const int64_t whole = n / Src::kPer;
+      const uint4* p = reinterpret_cast<const uint4*>(src.p);
+#pragma unroll 4
+      for (int64_t v = tid; v < whole; v += kCompactThreads) {
+        const int c = src.count16(p[v]);
+        all += c;
+        before += v * Src::kPer < first ? c : 0;
+      }
+      done = whole * Src::kPer;
+    }
+#pragma unroll 4
+    for (int64_t i = done + tid; i < n; i += kCompactThreads) {
+      const int c = src(i) ? 1 : 0;
+      all += c;
+      before += i < first ? c : 0;
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      all += __shfl_xor(all, off);
+      before += __shfl_xor(before, off);
+    }
+  }
+  if (lane == 0) {
+    s_own[wave] = own;
+    s_before[wave] = before;
+    s_all[wave] = all;
+  }
+  __syncthreads();
+  int64_t full_before = 0, nf = 0;
+#pragma unroll
+  for (int w = 0; w < kCompactWaves; ++w) {
+    full_before += s_before[w] + (w < wave ? s_own[w] : 0);
+    nf += gridDim.x > 1 ? s_all[w] : s_own[w];
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    counts[0] = static_cast<int32_t>(nf);
+    counts[1] = static_cast<int32_t>(n - nf);
+  }
+  compact_write<kWholeGroups>(bal, full_before, nf, n, indices);
 }
 
 template <typename Src>
@@ -74,7 +197,7 @@ __global__ __launch_bounds__(kCompactThreads) void compact_count_kernel(
   int cnt = 0;
 #pragma unroll
   for (int e = 0; e < kCompactGroups; ++e) {
-    const int64_t i = compact_elem(wave, e, lane);
+    const int64_t i = compact_elem<kCompactGroups>(wave, e, lane);
     const bool f = i < n && src(i);
     cnt += __builtin_popcountll(wave_ballot(f));
   }
@@ -87,7 +210,6 @@ __global__ __launch_bounds__(kCompactThreads) void compact_count_kernel(
   }
 }
 
-// block_counts == nullptr: a single block covers the whole mask.
 template <typename Src>
 __global__ __launch_bounds__(kCompactThreads) void compact_scatter_kernel(
     const Src src, int64_t n, const int32_t* __restrict__ block_counts,
@@ -99,7 +221,7 @@ __global__ __launch_bounds__(kCompactThreads) void compact_scatter_kernel(
   int cnt = 0;
 #pragma unroll
   for (int e = 0; e < kCompactGroups; ++e) {
-    const int64_t i = compact_elem(wave, e, lane);
+    const int64_t i = compact_elem<kCompactGroups>(wave, e, lane);
     const bool f = i < n && src(i);
     bal[e] = wave_ballot(f);
     cnt += __builtin_popcountll(bal[e]);
@@ -107,17 +229,15 @@ __global__ __launch_bounds__(kCompactThreads) void compact_scatter_kernel(
   if (lane == 0) s_wave[wave] = cnt;
   if (wave == 0) {
     int pre = 0, tot = 0;
-    if (block_counts != nullptr) {
-      for (int j = lane; j < nblocks; j += 64) {
-        const int c = block_counts[j];
-        tot += c;
-        pre += (j < static_cast<int>(blockIdx.x)) ? c : 0;
-      }
+    for (int j = lane; j < nblocks; j += 64) {
+      const int c = block_counts[j];
+      tot += c;
+      pre += (j < static_cast<int>(blockIdx.x)) ? c : 0;
+    }
 #pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) {
-        pre += __shfl_xor(pre, off);
-        tot += __shfl_xor(tot, off);
-      }
+    for (int off = 32; off >= 1; off >>= 1) {
+      pre += __shfl_xor(pre, off);
+      tot += __shfl_xor(tot, off);
     }
     if (lane == 0) {
       s_prefix = pre;
@@ -125,31 +245,14 @@ __global__ __launch_bounds__(kCompactThreads) void compact_scatter_kernel(
     }
   }
   __syncthreads();
-  int wave_prefix = s_prefix, block_total = 0;
-  for (int w = 0; w < kCompactWaves; ++w) {
-    const int c = s_wave[w];
-    wave_prefix += (w < wave) ? c : 0;
-    block_total += c;
-  }
-  const int64_t nf = (block_counts != nullptr) ? s_total : block_total;
+  int wave_prefix = s_prefix;
+  for (int w = 0; w < wave; ++w) wave_prefix += s_wave[w];
+  const int64_t nf = s_total;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     counts[0] = static_cast<int32_t>(nf);
     counts[1] = static_cast<int32_t>(n - nf);
   }
-  int64_t full_before = wave_prefix;
-#pragma unroll
-  for (int e = 0; e < kCompactGroups; ++e) {
-    const int64_t i = compact_elem(wave, e, lane);
-    const uint64_t b = bal[e];
-    const int64_t fb = full_before + count_below(b);
-    if (i < n) {
-      if ((b >> lane) & 1ull)
-        indices[fb] = static_cast<int32_t>(i);
-      else
-        indices[nf + (i - fb)] = static_cast<int32_t>(i);
-    }
-    full_before += __builtin_popcountll(b);
-  }
+  compact_write<kCompactGroups>(bal, wave_prefix, nf, n, indices);
 }
 
 // ---------------------------------------------------------------------------
@@ -346,14 +449,25 @@ int compact_impl(const Src& src, bool src_null, int64_t n, int32_t* indices, int
       return SWATTN_EWORKSPACE;
     }
     if (!aligned256(workspace)) return invalid(std::string(name) + ": workspace must be 256-byte aligned");
+  }
+  // Masks of up to kWholeBytes (kWholeUnaligned positions where 16-byte loads
+  // cannot be used) go through one kernel whose blocks each read all of it;
+  // beyond that those reads take longer than a second launch.
+  const bool vec = aligned16(src.p);
+  if (vec ? n * 16 <= kWholeBytes * Src::kPer : n <= kWholeUnaligned) {
+    const dim3 grid(static_cast<uint32_t>(ceil_div(n, kWholeChunk)));
+    if (vec)
+      hipLaunchKernelGGL((compact_whole_kernel<Src, true>), grid, dim3(kCompactThreads), 0, st, src,
+                         n, indices, counts);
+    else
+      hipLaunchKernelGGL((compact_whole_kernel<Src, false>), grid, dim3(kCompactThreads), 0, st, src,
+                         n, indices, counts);
+  } else {
     int32_t* bc = static_cast<int32_t*>(workspace);
     hipLaunchKernelGGL(compact_count_kernel<Src>, dim3(nb), dim3(kCompactThreads), 0, st, src, n,
                        bc);
     hipLaunchKernelGGL(compact_scatter_kernel<Src>, dim3(nb), dim3(kCompactThreads), 0, st, src,
                        n, static_cast<const int32_t*>(bc), static_cast<int>(nb), indices, counts);
-  } else {
-    hipLaunchKernelGGL(compact_scatter_kernel<Src>, dim3(1), dim3(kCompactThreads), 0, st, src, n,
-                       static_cast<const int32_t*>(nullptr), 1, indices, counts);
   }
   return launch_status(name);
 }
