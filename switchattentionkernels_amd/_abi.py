@@ -46,6 +46,13 @@ SIGNATURES = {
                                           _i32, _i32, ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
 }
 
+# Entry points of libswattn.so for this package only (csrc/swattn_internal.h).
+INTERNAL_SIGNATURES = {
+    "swattn_build_metadata_host": (ctypes.c_int, [_vp, _vp, _i32, _i64, _i64, _i32,
+                                                  _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "swattn_check_bounds": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp]),
+}
+
 # libswattn_probe.so (bench.py's measurement probe; not part of swattn.h).
 PROBE_SIGNATURES = {
     "swattn_mfma_peak": (ctypes.c_int, [_i64, _i32, _vp, _vp]),

@@ -14,7 +14,7 @@ import threading
 
 import torch  # noqa: F401  -- loads PyTorch's HIP runtime before the library
 
-from ._abi import PROBE_SIGNATURES, SIGNATURES, bind  # noqa: F401  -- part of this module's API
+from ._abi import INTERNAL_SIGNATURES, PROBE_SIGNATURES, SIGNATURES, bind  # noqa: F401  -- API
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libswattn.so")
@@ -40,7 +40,7 @@ def lib() -> ctypes.CDLL:
                 raise LibraryNotBuilt(
                     f"{LIB_PATH} is missing: build it with "
                     "`python -m switchattentionkernels_amd.build`")
-            _lib = bind(ctypes.CDLL(LIB_PATH))
+            _lib = bind(bind(ctypes.CDLL(LIB_PATH)), INTERNAL_SIGNATURES)
     return _lib
 
 

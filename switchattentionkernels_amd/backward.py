@@ -36,14 +36,16 @@ def _check_monotone(metadata: SwitchAttentionMetadata, full: torch.Tensor,
     every single causal sequence and for packed sequences in order).  A
     start past its row's end is an empty range and counts as the end, as in
     the kernels.  One device-to-host read."""
-    ok = torch.ones((), dtype=torch.bool, device=full.device)
-    for lst, starts in ((full, metadata.full_starts), (local, metadata.local_starts)):
-        if lst.numel() > 1:
-            li = lst.long()
-            ends = metadata.causal_ends[li]
-            for b in (torch.minimum(starts[li], ends), ends):
-                ok = ok & (b[1:] >= b[:-1]).all()
-    if not bool(ok.item()):
+    dev = full.device
+    flags = torch.empty(1, dtype=torch.int32, device=dev)
+    with _lib.on_device(dev):
+        st = _lib.lib().swattn_check_bounds(
+            full.data_ptr(), full.numel(), local.data_ptr(), local.numel(),
+            metadata.full_starts.data_ptr(), metadata.local_starts.data_ptr(),
+            metadata.causal_ends.data_ptr(), metadata.causal_ends.numel(), flags.data_ptr(),
+            _lib.stream_handle(dev))
+    _lib.check(st, "swattn_check_bounds")
+    if flags.item():
         raise ValueError(MSG_META + ": key bounds must be non-decreasing along each index list "
                          "for the backward pass")
 

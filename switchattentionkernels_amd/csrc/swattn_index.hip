@@ -4,10 +4,12 @@
 // Reference tags: V = swiattn_gqa_prefill_varlen.py, F = swiattn_gqa_prefill.py.
 
 #include <limits.h>
+#include <string.h>
 
 #include <string>
 
 #include "common.h"
+#include "swattn_internal.h"
 
 namespace swattn {
 
@@ -311,31 +313,97 @@ __device__ __forceinline__ int find_segment(const int32_t* cu, int nseq, int64_t
   return lo;
 }
 
-__global__ __launch_bounds__(256) void metadata_kernel(
-    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_kv, int nseq, int64_t total_q,
-    int64_t total_kv, int window, int32_t* __restrict__ q_pos, int32_t* __restrict__ kv_pos,
-    int32_t* __restrict__ q_seg, int32_t* __restrict__ kv_seg, int32_t* __restrict__ full_starts,
-    int32_t* __restrict__ local_starts, int32_t* __restrict__ causal_ends) {
+struct MetadataOut {
+  int32_t *q_pos, *kv_pos, *q_seg, *kv_seg, *full_starts, *local_starts, *causal_ends;
+};
+
+__device__ __forceinline__ void metadata_entry(const int32_t* cu_q, const int32_t* cu_kv, int nseq,
+                                               int64_t total_q, int64_t total_kv, int window,
+                                               const MetadataOut& o) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t < total_q) {
     const int s = find_segment(cu_q, nseq, t);
     const int64_t i = t - cu_q[s];
     const int64_t ks = cu_kv[s], klen = static_cast<int64_t>(cu_kv[s + 1]) - ks;
-    q_pos[t] = static_cast<int32_t>(i);
-    q_seg[t] = s;
-    full_starts[t] = static_cast<int32_t>(ks);
+    o.q_pos[t] = static_cast<int32_t>(i);
+    o.q_seg[t] = s;
+    o.full_starts[t] = static_cast<int32_t>(ks);
     const int64_t lo = i - window + 1;
-    local_starts[t] = static_cast<int32_t>(ks + (lo > 0 ? lo : 0));
-    causal_ends[t] = static_cast<int32_t>(ks + (i + 1 < klen ? i + 1 : klen));
+    o.local_starts[t] = static_cast<int32_t>(ks + (lo > 0 ? lo : 0));
+    o.causal_ends[t] = static_cast<int32_t>(ks + (i + 1 < klen ? i + 1 : klen));
   }
   if (t < total_kv) {
     const int s = find_segment(cu_kv, nseq, t);
-    kv_pos[t] = static_cast<int32_t>(t - cu_kv[s]);
-    kv_seg[t] = s;
+    o.kv_pos[t] = static_cast<int32_t>(t - cu_kv[s]);
+    o.kv_seg[t] = s;
   }
 }
 
+__global__ __launch_bounds__(256) void metadata_kernel(const int32_t* __restrict__ cu_q,
+                                                       const int32_t* __restrict__ cu_kv, int nseq,
+                                                       int64_t total_q, int64_t total_kv,
+                                                       int window, const MetadataOut o) {
+  metadata_entry(cu_q, cu_kv, nseq, total_q, total_kv, window, o);
+}
+
+// The same with the offsets as kernel arguments (up to kCuMax - 1 sequences),
+// staged in LDS for the searches.  The caller's offsets live on the host: as
+// device arrays they took two blocking copies of about 15 us before the launch.
+constexpr int kCuMax = 257;
+struct CuArgs {
+  int32_t q[kCuMax], kv[kCuMax];
+};
+static_assert(sizeof(CuArgs) <= 3072, "kernel arguments end at 4 KiB");
+__global__ __launch_bounds__(256) void metadata_args_kernel(const CuArgs cu, int nseq,
+                                                            int64_t total_q, int64_t total_kv,
+                                                            int window, const MetadataOut o) {
+  __shared__ int32_t s_q[kCuMax], s_kv[kCuMax];
+  for (int i = threadIdx.x; i <= nseq; i += 256) {
+    s_q[i] = cu.q[i];
+    s_kv[i] = cu.kv[i];
+  }
+  __syncthreads();
+  metadata_entry(s_q, s_kv, nseq, total_q, total_kv, window, o);
+}
+
+// Whether each list's key bounds are non-decreasing along it (a start past its
+// row's end counts as the end): what the backward's searches need.  One thread
+// per neighbouring pair of both lists; a listed position outside [0, total_q)
+// is never dereferenced and fails the check.
+__global__ __launch_bounds__(256) void check_bounds_kernel(
+    const int32_t* __restrict__ full, int64_t nf, const int32_t* __restrict__ local, int64_t nl,
+    const int32_t* __restrict__ full_starts, const int32_t* __restrict__ local_starts,
+    const int32_t* __restrict__ ends, int64_t total_q, int32_t* __restrict__ flags) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  auto falls = [&](const int32_t* list, int64_t n, const int32_t* starts) {
+    if (i + 1 >= n) return false;
+    const int32_t a = list[i], b = list[i + 1];
+    if (a < 0 || a >= total_q || b < 0 || b >= total_q) return true;
+    const int32_t ea = ends[a], eb = ends[b];
+    return eb < ea || min(starts[b], eb) < min(starts[a], ea);
+  };
+  const bool f = falls(full, nf, full_starts) || falls(local, nl, local_starts);
+  if (wave_ballot(f) != 0 && (threadIdx.x & 63) == 0) atomicOr(flags, 1);
+}
+
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+static_assert(kCuMax == SWATTN_METADATA_HOST_MAX_SEQS + 1, "offsets of the header's limit");
+
+// Argument checks shared by both metadata entry points.
+int metadata_check(const char* name, const int32_t* cu_q, const int32_t* cu_kv, int32_t num_seqs,
+                   int64_t total_q, int64_t total_kv, int32_t window, const MetadataOut& o) {
+  const std::string n(name);
+  if (num_seqs < 1 || total_q < 0 || total_kv < 0 || total_q > INT32_MAX || total_kv > INT32_MAX)
+    return invalid(n + ": bad sizes");
+  if (window <= 0) return invalid(n + ": window must be positive");
+  if (cu_q == nullptr || cu_kv == nullptr) return invalid(n + ": null cu_seqlens");
+  if ((total_q > 0 && (o.q_pos == nullptr || o.q_seg == nullptr || o.full_starts == nullptr ||
+                       o.local_starts == nullptr || o.causal_ends == nullptr)) ||
+      (total_kv > 0 && (o.kv_pos == nullptr || o.kv_seg == nullptr)))
+    return invalid(n + ": null output");
+  return SWATTN_OK;
+}
 
 template <typename Src>
 int compact_impl(const Src& src, bool src_null, int64_t n, int32_t* indices, int32_t* counts,
@@ -401,28 +469,64 @@ int swattn_check_indices(const int32_t* full, int64_t n_full, const int32_t* loc
   return launch_status("swattn_check_indices");
 }
 
+int swattn_check_bounds(const int32_t* full, int64_t n_full, const int32_t* local, int64_t n_local,
+                        const int32_t* full_starts, const int32_t* local_starts,
+                        const int32_t* causal_ends, int64_t total_q, int32_t* flags,
+                        void* stream) {
+  if (n_full < 0 || n_local < 0 || total_q < 0 || total_q > INT32_MAX)
+    return invalid("swattn_check_bounds: bad sizes");
+  if (flags == nullptr || (n_full > 0 && (full == nullptr || full_starts == nullptr)) ||
+      (n_local > 0 && (local == nullptr || local_starts == nullptr)) ||
+      (n_full + n_local > 0 && causal_ends == nullptr))
+    return invalid("swattn_check_bounds: null pointer");
+  const hipStream_t st = as_stream(stream);
+  hipLaunchKernelGGL(flags_clear_kernel, dim3(1), dim3(1), 0, st, flags);
+  const int64_t n = n_full > n_local ? n_full : n_local;
+  if (n > 1)
+    hipLaunchKernelGGL(check_bounds_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, st, full, n_full,
+                       local, n_local, full_starts, local_starts, causal_ends, total_q, flags);
+  return launch_status("swattn_check_bounds");
+}
+
 int swattn_build_metadata(const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
                           int32_t num_seqs, int64_t total_q, int64_t total_kv, int32_t window,
                           int32_t* q_positions, int32_t* kv_positions, int32_t* q_segment_ids,
                           int32_t* kv_segment_ids, int32_t* full_starts, int32_t* local_starts,
                           int32_t* causal_ends, void* stream) {
-  if (num_seqs < 1 || total_q < 0 || total_kv < 0 || total_q > INT32_MAX || total_kv > INT32_MAX)
-    return invalid("swattn_build_metadata: bad sizes");
-  if (window <= 0) return invalid("swattn_build_metadata: window must be positive");
-  if (cu_seqlens_q == nullptr || cu_seqlens_kv == nullptr)
-    return invalid("swattn_build_metadata: null cu_seqlens");
-  if ((total_q > 0 && (q_positions == nullptr || q_segment_ids == nullptr ||
-                       full_starts == nullptr || local_starts == nullptr ||
-                       causal_ends == nullptr)) ||
-      (total_kv > 0 && (kv_positions == nullptr || kv_segment_ids == nullptr)))
-    return invalid("swattn_build_metadata: null output");
+  const MetadataOut o{q_positions, kv_positions, q_segment_ids, kv_segment_ids,
+                      full_starts, local_starts, causal_ends};
+  const char* name = "swattn_build_metadata";
+  const int st = metadata_check(name, cu_seqlens_q, cu_seqlens_kv, num_seqs, total_q, total_kv,
+                                window, o);
+  const int64_t n = total_q > total_kv ? total_q : total_kv;
+  if (st != SWATTN_OK || n == 0) return st;
+  hipLaunchKernelGGL(metadata_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, as_stream(stream),
+                     cu_seqlens_q, cu_seqlens_kv, num_seqs, total_q, total_kv, window, o);
+  return launch_status(name);
+}
+
+int swattn_build_metadata_host(const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
+                               int32_t num_seqs, int64_t total_q, int64_t total_kv, int32_t window,
+                               int32_t* q_positions, int32_t* kv_positions,
+                               int32_t* q_segment_ids, int32_t* kv_segment_ids,
+                               int32_t* full_starts, int32_t* local_starts, int32_t* causal_ends,
+                               void* stream) {
+  const MetadataOut o{q_positions, kv_positions, q_segment_ids, kv_segment_ids,
+                      full_starts, local_starts, causal_ends};
+  const char* name = "swattn_build_metadata_host";
+  const int st = metadata_check(name, cu_seqlens_q, cu_seqlens_kv, num_seqs, total_q, total_kv,
+                                window, o);
+  if (st != SWATTN_OK) return st;
+  if (num_seqs > SWATTN_METADATA_HOST_MAX_SEQS)
+    return invalid("swattn_build_metadata_host: too many sequences (use swattn_build_metadata)");
   const int64_t n = total_q > total_kv ? total_q : total_kv;
   if (n == 0) return SWATTN_OK;
-  hipLaunchKernelGGL(metadata_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, as_stream(stream),
-                     cu_seqlens_q, cu_seqlens_kv, num_seqs, total_q, total_kv, window,
-                     q_positions, kv_positions, q_segment_ids, kv_segment_ids, full_starts,
-                     local_starts, causal_ends);
-  return launch_status("swattn_build_metadata");
+  CuArgs cu{};
+  memcpy(cu.q, cu_seqlens_q, (num_seqs + 1) * sizeof(int32_t));
+  memcpy(cu.kv, cu_seqlens_kv, (num_seqs + 1) * sizeof(int32_t));
+  hipLaunchKernelGGL(metadata_args_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, as_stream(stream),
+                     cu, num_seqs, total_q, total_kv, window, o);
+  return launch_status(name);
 }
 
 }  // extern "C"

@@ -16,11 +16,14 @@ packed sequence, so attention never crosses a sequence boundary.
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import torch
 
 from . import _lib
+
+HOST_MAX_SEQS = 256   # SWATTN_METADATA_HOST_MAX_SEQS
 
 
 @dataclass(frozen=True)
@@ -76,19 +79,27 @@ def build_switch_attention_metadata(q_len: int, kv_len: int, *, device, window_s
     ck = _as_cu(ck_src, kv_len, "cu_seqlens_kv")
     if len(ck) != len(cq):
         raise ValueError("cu_seqlens and cu_seqlens_kv must describe the same number of sequences")
-    cq_t = torch.tensor(cq, dtype=torch.int32, device=dev)
-    ck_t = torch.tensor(ck, dtype=torch.int32, device=dev)
-
-    def e(n):
-        return torch.empty(n, dtype=torch.int32, device=dev)
-
-    md = SwitchAttentionMetadata(e(q_len), e(kv_len), e(q_len), e(kv_len), e(q_len), e(q_len),
-                                 e(q_len))
+    if q_len == kv_len:
+        # One allocation; the fields are its rows.
+        md = SwitchAttentionMetadata(*torch.empty((7, q_len), dtype=torch.int32, device=dev)
+                                     .unbind(0))
+    else:
+        md = SwitchAttentionMetadata(*(torch.empty(n, dtype=torch.int32, device=dev) for n in
+                                       (q_len, kv_len, q_len, kv_len, q_len, q_len, q_len)))
+    L, nseq = _lib.lib(), len(cq) - 1
+    outs = [t.data_ptr() for t in (md.q_positions, md.kv_positions, md.q_segment_ids,
+                                   md.kv_segment_ids, md.full_starts, md.local_starts,
+                                   md.causal_ends)]
     with _lib.on_device(dev):
-        st = _lib.lib().swattn_build_metadata(
-            cq_t.data_ptr(), ck_t.data_ptr(), len(cq) - 1, q_len, kv_len, window_size,
-            md.q_positions.data_ptr(), md.kv_positions.data_ptr(), md.q_segment_ids.data_ptr(),
-            md.kv_segment_ids.data_ptr(), md.full_starts.data_ptr(), md.local_starts.data_ptr(),
-            md.causal_ends.data_ptr(), _lib.stream_handle(dev))
+        stream = _lib.stream_handle(dev)
+        if nseq <= HOST_MAX_SEQS:   # the offsets travel as kernel arguments
+            arr = ctypes.c_int32 * (nseq + 1)
+            st = L.swattn_build_metadata_host(arr(*cq), arr(*ck), nseq, q_len, kv_len,
+                                              window_size, *outs, stream)
+        else:
+            cq_t = torch.tensor(cq, dtype=torch.int32, device=dev)
+            ck_t = torch.tensor(ck, dtype=torch.int32, device=dev)
+            st = L.swattn_build_metadata(cq_t.data_ptr(), ck_t.data_ptr(), nseq, q_len, kv_len,
+                                         window_size, *outs, stream)
     _lib.check(st, "swattn_build_metadata")
     return md
