@@ -1,4 +1,5 @@
-"""ctypes binding of ``libswattn.so`` (declared in ``include/swattn.h``).
+"""Bindings of ``libswattn.so``: ctypes for the C ABI (``include/swattn.h``) and
+the native extension for the hot calls (``csrc/native.cpp``).
 
 The library is built in-tree by ``switchattentionkernels_amd.build``.  There
 is no fallback: if the library is missing every call raises, so a GPU run can
@@ -9,6 +10,8 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -18,10 +21,12 @@ from ._abi import INTERNAL_SIGNATURES, PROBE_SIGNATURES, SIGNATURES, bind  # noq
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libswattn.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 PROBE_PATH = os.path.join(_HERE, "libswattn_probe.so")
 
 _lock = threading.Lock()
 _lib = None
+_native = None
 _probe = None
 
 
@@ -42,6 +47,28 @@ def lib() -> ctypes.CDLL:
                     "`python -m switchattentionkernels_amd.build`")
             _lib = bind(bind(ctypes.CDLL(LIB_PATH)), INTERNAL_SIGNATURES)
     return _lib
+
+
+def native():
+    """Load (once) and return the extension with the hot calls' host path
+    (``csrc/native.cpp``), which calls the library loaded by ``lib()``."""
+    global _native
+    if _native is not None:
+        return _native
+    lib()
+    with _lock:
+        if _native is None:
+            if not os.path.exists(NATIVE_PATH):
+                raise LibraryNotBuilt(
+                    f"{NATIVE_PATH} is missing: build it with "
+                    "`python -m switchattentionkernels_amd.build`")
+            spec = importlib.util.spec_from_file_location(
+                "_native", NATIVE_PATH,
+                loader=importlib.machinery.ExtensionFileLoader("_native", NATIVE_PATH))
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            _native = mod
+    return _native
 
 
 def probe_lib() -> ctypes.CDLL:

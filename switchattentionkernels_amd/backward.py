@@ -25,7 +25,7 @@ import torch
 
 from . import _lib
 from .metadata import SwitchAttentionMetadata, build_switch_attention_metadata
-from .prefill import (LOG2E, MSG_META, _check_lists, _check_metadata, _validate_qkv,
+from .prefill import (LOG2E, MSG_META, _check_lists, _check_metadata, check_qkv,
                       switch_gqa_prefill_forward)
 
 
@@ -71,7 +71,7 @@ def switch_gqa_prefill_backward(
     Returns ``(dq, dk, dv)`` in bf16; a query row that sees no key gets
     ``dq = 0`` and a key row that no query sees gets ``dk = dv = 0``.
     """
-    _validate_qkv(q, k, v)
+    check_qkv(q, k, v)
     if window_size <= 0:
         raise ValueError("window_size must be positive")
     for name, t, dt in (("output", output, torch.bfloat16), ("grad_output", grad_output,
@@ -81,8 +81,8 @@ def switch_gqa_prefill_backward(
     if (lse.shape != q.shape[:3] or lse.dtype != torch.float32 or lse.device != q.device
             or not lse.is_contiguous()):
         raise ValueError("lse must be a contiguous FP32 tensor shaped [B, Sq, Hq]")
-    batch, q_len, heads, dim = (int(x) for x in q.shape)
-    kv_len, kv_heads = int(k.shape[1]), int(k.shape[2])
+    batch, q_len, _, dim = q.shape
+    kv_len = k.shape[1]
     if metadata is not None and batch != 1:
         raise ValueError("position metadata requires batch size 1; pack sequences with cu_seqlens")
     total_q = batch * q_len
@@ -94,30 +94,12 @@ def switch_gqa_prefill_backward(
     scale = ((1.0 / dim) ** 0.5 if sm_scale is None else float(sm_scale))
     if not scale > 0:
         raise ValueError("sm_scale must be positive")
-    # The lists cover every query position once (checked above), and the
-    # kernels write every listed row (0 for a row with no key): no fill.
-    dq = torch.empty_like(q)
-    dk = torch.empty_like(k)
-    dv = torch.empty_like(v)
-    md = metadata
-    L = _lib.lib()
-    ws_bytes = int(L.swattn_prefill_bwd_workspace_bytes(batch, kv_len, heads, kv_heads, dim,
-                                                        int(window_size), full.numel(),
-                                                        local.numel()))
-    workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
+    fs, ls, ends = (None, None, None) if metadata is None else (
+        metadata.full_starts, metadata.local_starts, metadata.causal_ends)
     with _lib.on_device(q.device):
-        st = L.swattn_prefill_bwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), output.data_ptr(), lse.data_ptr(),
-            grad_output.data_ptr(), full.data_ptr(), full.numel(), local.data_ptr(),
-            local.numel(),
-            _lib.ptr(md.full_starts) if md is not None else None,
-            _lib.ptr(md.local_starts) if md is not None else None,
-            _lib.ptr(md.causal_ends) if md is not None else None,
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), batch, q_len, kv_len, heads, kv_heads,
-            dim, int(window_size), scale * LOG2E, workspace.data_ptr(), ws_bytes,
-            _lib.stream_handle(q.device))
-    _lib.check(st, "swattn_prefill_bwd")
-    return dq, dk, dv
+        return _lib.native().prefill_backward(q, k, v, output, lse, grad_output, full, local, fs,
+                                              ls, ends, int(window_size), scale * LOG2E,
+                                              _lib.stream_handle(q.device))
 
 
 class SwitchGQAPrefillFunction(torch.autograd.Function):
@@ -133,11 +115,14 @@ class SwitchGQAPrefillFunction(torch.autograd.Function):
         ctx.window_size = window_size
         ctx.sm_scale = sm_scale
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)   # no zeros for lse's gradient, which is never used
         return out, lse
 
     @staticmethod
     def backward(ctx, grad_out, grad_lse):
         q, k, v, out, lse, full, local = ctx.saved_tensors
+        if grad_out is None:
+            grad_out = torch.zeros_like(out)
         g = grad_out.to(torch.bfloat16).contiguous()
         dq, dk, dv = switch_gqa_prefill_backward(q, k, v, out, lse, g, full, local,
                                                  metadata=ctx.md,
@@ -161,7 +146,7 @@ def switch_gqa_prefill_varlen(q, k, v, full_query_indices, local_query_indices, 
     """``switch_gqa_prefill_varlen_forward`` with autograd support for q, k, v:
     ``q``/``k``/``v`` are ``[1, T, H, 128]`` with the sequences concatenated
     along T at offsets ``cu_seqlens``."""
-    _validate_qkv(q, k, v)
+    check_qkv(q, k, v)
     md = build_switch_attention_metadata(int(q.shape[1]), int(k.shape[1]), device=q.device,
                                          window_size=window_size, cu_seqlens=cu_seqlens,
                                          cu_seqlens_kv=cu_seqlens_kv)

@@ -110,6 +110,37 @@ def build_probe(verbose: bool = False) -> str:
     return build(verbose=verbose, out=PROBE_LIB, sources=PROBE_SOURCES)
 
 
+NATIVE_LIB = os.path.join(HERE, "_native.so")
+
+
+def build_native(verbose: bool = False) -> str:
+    """Compile ``_native.so``, the extension with the hot calls' host path
+    (``csrc/native.cpp``, host code only), against torch and the
+    ``libswattn.so`` next to it (built first)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    tl = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = NATIVE_LIB + ".tmp"
+    cmd = [os.environ.get("CXX") or shutil.which("g++") or "c++", "-O2", "-std=c++17", "-shared",
+           "-fPIC", "-fvisibility=hidden", "-DTORCH_EXTENSION_NAME=_native",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I", os.path.join(ROOT, "include"), "-I", CSRC]
+    for p in include_paths() + [sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", p]
+    cmd += [os.path.join(CSRC, "native.cpp"), "-o", tmp, "-L", tl, "-ltorch", "-ltorch_cpu",
+            "-lc10", "-ltorch_python", "-L", HERE, "-lswattn", "-Wl,-rpath," + tl,
+            "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compiling native.cpp failed ({res.returncode}):\n{res.stderr}")
+    os.replace(tmp, NATIVE_LIB)
+    return NATIVE_LIB
+
+
 C_CALLER_SRC = os.path.join(ROOT, "tests", "c_abi", "prefill_caller.cpp")
 C_CALLER = os.path.join(ROOT, "tests", "c_abi", "prefill_caller")
 
@@ -134,5 +165,6 @@ def build_c_caller(verbose: bool = False) -> str:
 
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_native(verbose=True))
     print(build_probe(verbose=True))
     print(build_c_caller(verbose=True))

@@ -6,6 +6,8 @@
 #include <limits.h>
 #include <string.h>
 
+#include <atomic>
+#include <chrono>
 #include <string>
 
 #include "common.h"
@@ -131,7 +133,13 @@ constexpr int kWholeGroups = 4;
 constexpr int kWholeChunk = kCompactThreads * kWholeGroups;   // 4096 positions per block
 constexpr int64_t kWholeBytes = 256 << 10;   // a block reads at most this much (10 us, as two kernels)
 constexpr int64_t kWholeUnaligned = 64 << 10;   // positions, read one by one (8 us; 131072: 12)
-template <typename Src, bool kVec>
+static_assert(kWholeBytes / kWholeChunk + 2 <= SWATTN_COMPACT_HOST_WORDS, "one word per block");
+//
+// kHost: counts is pinned host memory that a host thread polls, with one word
+// per block after the counts.  A block sets its word when its indices are in
+// memory (system-scope release), so that a host that has seen all of them may
+// hand the lists to any stream, as after a synchronisation.
+template <typename Src, bool kVec, bool kHost>
 __global__ __launch_bounds__(kCompactThreads) void compact_whole_kernel(
     const Src src, int64_t n, int32_t* __restrict__ indices, int32_t* __restrict__ counts) {
   __shared__ int s_own[kCompactWaves], s_before[kCompactWaves], s_all[kCompactWaves];
@@ -189,6 +197,12 @@ __global__ __launch_bounds__(kCompactThreads) void compact_whole_kernel(
     counts[1] = static_cast<int32_t>(n - nf);
   }
   compact_write<kWholeGroups>(bal, full_before, nf, n, indices);
+  if constexpr (kHost) {
+    __threadfence_system();   // every wave's own stores
+    __syncthreads();
+    if (tid == 0)
+      __hip_atomic_store(counts + 2 + blockIdx.x, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 template <typename Src>
@@ -388,6 +402,10 @@ __global__ __launch_bounds__(256) void check_bounds_kernel(
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+int compact_logits_impl(const void* logits, int32_t dtype, int64_t n, float threshold,
+                        int32_t* indices, int32_t* counts, void* workspace, size_t workspace_bytes,
+                        void* stream, const char* name, int* host_blocks);
+
 static_assert(kCuMax == SWATTN_METADATA_HOST_MAX_SEQS + 1, "offsets of the header's limit");
 
 // Argument checks shared by both metadata entry points.
@@ -407,7 +425,8 @@ int metadata_check(const char* name, const int32_t* cu_q, const int32_t* cu_kv, 
 
 template <typename Src>
 int compact_impl(const Src& src, bool src_null, int64_t n, int32_t* indices, int32_t* counts,
-                 void* workspace, size_t workspace_bytes, void* stream, const char* name);
+                 void* workspace, size_t workspace_bytes, void* stream, const char* name,
+                 int* host_blocks = nullptr);
 
 }  // namespace
 }  // namespace swattn
@@ -435,23 +454,73 @@ int swattn_compact_logits(const void* logits, int32_t dtype, int64_t n, float th
                           int32_t* indices, int32_t* counts, void* workspace,
                           size_t workspace_bytes, void* stream) {
   const char* name = "swattn_compact_logits";
+  return compact_logits_impl(logits, dtype, n, threshold, indices, counts, workspace,
+                             workspace_bytes, stream, name, nullptr);
+}
+
+int swattn_compact_wait(const void* x, int32_t dtype, int64_t n, float threshold, int32_t* indices,
+                        int32_t* host, void* workspace, size_t workspace_bytes, void* stream) {
+  const char* name = dtype < 0 ? "swattn_compact" : "swattn_compact_logits";
+  if (host == nullptr) return invalid(std::string(name) + ": null pointer");
+  for (int i = 0; i < SWATTN_COMPACT_HOST_WORDS; ++i) host[i] = 0;
+  int blocks = 0;
+  const int status =
+      dtype < 0 ? compact_impl(MaskSource{static_cast<const uint8_t*>(x)}, x == nullptr, n, indices,
+                               host, workspace, workspace_bytes, stream, name, &blocks)
+                : compact_logits_impl(x, dtype, n, threshold, indices, host, workspace,
+                                      workspace_bytes, stream, name, &blocks);
+  if (status != SWATTN_OK) return status;
+  // Poll the blocks' words for a while; then, or where none report, wait for
+  // the stream (it may hold any amount of earlier work, or have failed).
+  volatile int32_t* word = host + 2;
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int done = 0; blocks > 0;) {
+    while (done < blocks && word[done] != 0) ++done;
+    if (done == blocks) {
+      std::atomic_thread_fence(std::memory_order_acquire);
+      return SWATTN_OK;
+    }
+    __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) break;
+  }
+  const hipError_t e = hipStreamSynchronize(as_stream(stream));
+  if (e != hipSuccess) {
+    set_error(std::string(name) + ": " + hipGetErrorString(e));
+    return static_cast<int>(e);
+  }
+  return SWATTN_OK;
+}
+
+}  // extern "C"
+
+namespace swattn {
+namespace {
+
+int compact_logits_impl(const void* logits, int32_t dtype, int64_t n, float threshold,
+                        int32_t* indices, int32_t* counts, void* workspace, size_t workspace_bytes,
+                        void* stream, const char* name, int* host_blocks) {
   switch (dtype) {
     case SWATTN_DTYPE_F32:
       return compact_impl(F32LogitSource{static_cast<const float*>(logits), threshold},
                           logits == nullptr, n, indices, counts, workspace, workspace_bytes,
-                          stream, name);
+                          stream, name, host_blocks);
     case SWATTN_DTYPE_BF16:
       return compact_impl(BF16LogitSource{static_cast<const uint16_t*>(logits), threshold},
                           logits == nullptr, n, indices, counts, workspace, workspace_bytes,
-                          stream, name);
+                          stream, name, host_blocks);
     case SWATTN_DTYPE_F16:
       return compact_impl(F16LogitSource{static_cast<const _Float16*>(logits), threshold},
                           logits == nullptr, n, indices, counts, workspace, workspace_bytes,
-                          stream, name);
+                          stream, name, host_blocks);
     default:
       return invalid("swattn_compact_logits: dtype must be SWATTN_DTYPE_F32, _BF16 or _F16");
   }
 }
+
+}  // namespace
+}  // namespace swattn
+
+extern "C" {
 
 int swattn_check_indices(const int32_t* full, int64_t n_full, const int32_t* local,
                          int64_t n_local, int64_t seq_len, int32_t* flags, void* stream) {
@@ -534,9 +603,12 @@ int swattn_build_metadata_host(const int32_t* cu_seqlens_q, const int32_t* cu_se
 namespace swattn {
 namespace {
 
+// host_blocks: counts is pinned host memory; set to the blocks that report
+// there (0: the stream has to be synchronised instead).
 template <typename Src>
 int compact_impl(const Src& src, bool src_null, int64_t n, int32_t* indices, int32_t* counts,
-                 void* workspace, size_t workspace_bytes, void* stream, const char* name) {
+                 void* workspace, size_t workspace_bytes, void* stream, const char* name,
+                 int* host_blocks) {
   if (n < 0 || n > INT32_MAX) return invalid(std::string(name) + ": n must be in [0, 2^31)");
   if (counts == nullptr || (n > 0 && (src_null || indices == nullptr)))
     return invalid(std::string(name) + ": null pointer");
@@ -560,12 +632,11 @@ int compact_impl(const Src& src, bool src_null, int64_t n, int32_t* indices, int
   const bool vec = aligned16(src.p);
   if (vec ? n * 16 <= kWholeBytes * Src::kPer : n <= kWholeUnaligned) {
     const dim3 grid(static_cast<uint32_t>(ceil_div(n, kWholeChunk)));
-    if (vec)
-      hipLaunchKernelGGL((compact_whole_kernel<Src, true>), grid, dim3(kCompactThreads), 0, st, src,
-                         n, indices, counts);
-    else
-      hipLaunchKernelGGL((compact_whole_kernel<Src, false>), grid, dim3(kCompactThreads), 0, st, src,
-                         n, indices, counts);
+    const auto kernel = host_blocks != nullptr
+                            ? (vec ? compact_whole_kernel<Src, true, true> : compact_whole_kernel<Src, false, true>)
+                            : (vec ? compact_whole_kernel<Src, true, false> : compact_whole_kernel<Src, false, false>);
+    if (host_blocks != nullptr) *host_blocks = static_cast<int>(grid.x);
+    hipLaunchKernelGGL(kernel, grid, dim3(kCompactThreads), 0, st, src, n, indices, counts);
   } else {
     int32_t* bc = static_cast<int32_t*>(workspace);
     hipLaunchKernelGGL(compact_count_kernel<Src>, dim3(nb), dim3(kCompactThreads), 0, st, src, n,

@@ -10,6 +10,18 @@ extern "C" {
 #endif
 
 /*
+ * swattn_compact (dtype -1: x is a byte mask) or swattn_compact_logits, waiting
+ * for the result: on return the lists are complete, for any stream, and host[0]
+ * and host[1] hold the counts.
+ *   host  SWATTN_COMPACT_HOST_WORDS int32 of pinned host memory, one call at a
+ *         time.  The kernel reports there; a device copy of the counts and a
+ *         stream synchronisation would take about 8 us more.
+ */
+#define SWATTN_COMPACT_HOST_WORDS 66
+int swattn_compact_wait(const void* x, int32_t dtype, int64_t n, float threshold, int32_t* indices,
+                        int32_t* host, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * swattn_build_metadata with the offsets in host memory (read before the call
  * returns, so that no device copy of them is needed), for up to
  * SWATTN_METADATA_HOST_MAX_SEQS sequences.  They must be ascending and end at

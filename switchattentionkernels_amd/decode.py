@@ -64,19 +64,11 @@ def switch_gqa_decode_forward(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     if not (k_cache.device == v_cache.device == dev):
         raise ValueError("Q and KV cache must be on the same device")
     scale = ((1.0 / dim) ** 0.5 if sm_scale is None else float(sm_scale)) * LOG2E
-    out = torch.empty_like(q)
-    lse = torch.empty(q.shape[:3], dtype=torch.float32, device=dev)
     lens = cache_lens.contiguous()
-    full = full_mask.contiguous().view(torch.uint8)
-    L = _lib.lib()
-    ws_bytes = int(L.swattn_decode_workspace_bytes(batch, cache_len, heads, kv_heads))
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    full = full_mask.contiguous()
     with _lib.on_device(dev):
-        st = L.swattn_decode_fwd(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-                                 lens.data_ptr(), full.data_ptr(), out.data_ptr(), lse.data_ptr(),
-                                 batch, cache_len, heads, kv_heads, dim, int(window_size), scale,
-                                 ws.data_ptr(), ws_bytes, _lib.stream_handle(dev))
-    _lib.check(st, "swattn_decode_fwd")
+        out, lse = _lib.native().decode_forward(q, k_cache, v_cache, lens, full, int(window_size),
+                                                scale, _lib.stream_handle(dev))
     if squeeze:
         return out[:, 0], lse[:, 0]
     return out, lse

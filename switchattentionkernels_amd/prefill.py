@@ -64,6 +64,12 @@ def _validate_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
         raise ValueError("Q/K/V must be on the same device")
 
 
+def check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
+    """``_validate_qkv``, in Python only where one of its conditions fails."""
+    if not _lib.native().qkv_ok(q, k, v):
+        _validate_qkv(q, k, v)
+
+
 def _prepare_indices(indices: torch.Tensor, *, device: torch.device) -> torch.Tensor:
     """Host-side part of V:271-286: shape, device and int32 cast.
 
@@ -202,17 +208,8 @@ def build_switch_query_indices(full_mask: torch.Tensor) -> Tuple[torch.Tensor, t
         raise ValueError("full_mask must hold fewer than 2^31 positions")
     dev = full_mask.device
     mask = full_mask.contiguous()
-    out = torch.empty(n, dtype=torch.int32, device=dev)
-    counts = torch.empty(2, dtype=torch.int32, device=dev)
-    L = _lib.lib()
-    ws_bytes = int(L.swattn_compact_workspace_bytes(n))
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     with _lib.on_device(dev):
-        st = L.swattn_compact(mask.data_ptr(), n, out.data_ptr(), counts.data_ptr(),
-                              ws.data_ptr(), ws_bytes, _lib.stream_handle(dev))
-    _lib.check(st, "swattn_compact")
-    nf = int(counts[0].item())
-    full, local = out[:nf], out[nf:]
+        full, local = _lib.native().compact(mask, -1, 0.0, _lib.stream_handle(dev))
     _tag_compacted(full, local, n)
     return full, local
 
@@ -245,19 +242,12 @@ def build_switch_query_indices_from_logits(
         raise ValueError("router_logits must hold fewer than 2^31 positions")
     dev = router_logits.device
     logits = router_logits.contiguous()
-    thr = float(torch.tensor(float(threshold), dtype=logits.dtype).item())
-    out = torch.empty(n, dtype=torch.int32, device=dev)
-    counts = torch.empty(2, dtype=torch.int32, device=dev)
-    L = _lib.lib()
-    ws_bytes = int(L.swattn_compact_workspace_bytes(n))
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
+    thr = float(threshold)
+    if thr != 0.0 and logits.dtype != torch.float32:   # fp32 is rounded by the call
+        thr = float(torch.tensor(thr, dtype=logits.dtype).item())
     with _lib.on_device(dev):
-        st = L.swattn_compact_logits(logits.data_ptr(), _LOGIT_DTYPES[logits.dtype], n, thr,
-                                     out.data_ptr(), counts.data_ptr(), ws.data_ptr(), ws_bytes,
-                                     _lib.stream_handle(dev))
-    _lib.check(st, "swattn_compact_logits")
-    nf = int(counts[0].item())
-    full, local = out[:nf], out[nf:]
+        full, local = _lib.native().compact(logits, _LOGIT_DTYPES[logits.dtype], thr,
+                                            _lib.stream_handle(dev))
     _tag_compacted(full, local, n)
     return full, local
 
@@ -288,11 +278,11 @@ def switch_gqa_prefill_forward(
     compatibility; values other than the reference's qualified schedule raise
     ``AssertionError`` as the reference kernel does (V:67-71).
     """
-    _validate_qkv(q, k, v)
+    check_qkv(q, k, v)
     if window_size <= 0:
         raise ValueError("window_size must be positive")
-    batch, q_len, heads, dim = (int(x) for x in q.shape)
-    kv_len, kv_heads = int(k.shape[1]), int(k.shape[2])
+    batch, q_len, _, dim = q.shape
+    kv_len = k.shape[1]
     if metadata is not None and batch != 1:
         raise ValueError("position metadata requires batch size 1; pack sequences with cu_seqlens")
     if kv_len == 0 and q_len > 0:
@@ -302,35 +292,19 @@ def switch_gqa_prefill_forward(
         _check_metadata(metadata, q_len, kv_len, q.device)
     full, local = _check_lists(full_query_indices, local_query_indices, total_q, q.device)
 
-    output = torch.empty_like(q)
-    lse = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
     if total_q == 0:
-        return output, lse
+        return (torch.empty_like(q),
+                torch.empty(q.shape[:3], dtype=torch.float32, device=q.device))
     assert block_m == 64, "the qualified schedule is BM64"
     assert block_k == 64, "the qualified schedule is BK64"
     assert num_stages == 1, "the qualified schedule uses one stage"
     assert threads == 128, "the qualified schedule uses 128 threads"
     scale = ((1.0 / dim) ** 0.5 if sm_scale is None else float(sm_scale)) * LOG2E
-    md = metadata
-    L = _lib.lib()
-    # The larger workspace that lets the kernel split long full items by key
-    # range when they would otherwise set its length (few KV heads).
-    ws_bytes = int(L.swattn_prefill_split_workspace_bytes(batch, q_len, kv_len, heads, kv_heads,
-                                                          dim, int(window_size), full.numel(),
-                                                          local.numel()))
-    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+    fs, ls, ends = (None, None, None) if metadata is None else (
+        metadata.full_starts, metadata.local_starts, metadata.causal_ends)
     with _lib.on_device(q.device):
-        st = L.swattn_prefill_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(),
-            full.data_ptr(), full.numel(), local.data_ptr(), local.numel(),
-            _lib.ptr(md.full_starts) if md is not None else None,
-            _lib.ptr(md.local_starts) if md is not None else None,
-            _lib.ptr(md.causal_ends) if md is not None else None,
-            output.data_ptr(), lse.data_ptr(), batch, q_len, kv_len, heads, kv_heads, dim,
-            int(window_size), scale, workspace.data_ptr(), ws_bytes,
-            _lib.stream_handle(q.device))
-    _lib.check(st, "swattn_prefill_fwd")
-    return output, lse
+        return _lib.native().prefill_forward(q, k, v, full, local, fs, ls, ends, int(window_size),
+                                             scale, _lib.stream_handle(q.device))
 
 
 def switch_gqa_prefill_varlen_forward(
@@ -349,7 +323,7 @@ def switch_gqa_prefill_varlen_forward(
     the sequences concatenated along T at offsets ``cu_seqlens``.  Builds the
     position metadata (``build_switch_attention_metadata``) and calls
     ``switch_gqa_prefill_forward``; attention never crosses a sequence."""
-    _validate_qkv(q, k, v)
+    check_qkv(q, k, v)
     md = build_switch_attention_metadata(int(q.shape[1]), int(k.shape[1]), device=q.device,
                                          window_size=window_size, cu_seqlens=cu_seqlens,
                                          cu_seqlens_kv=cu_seqlens_kv)
