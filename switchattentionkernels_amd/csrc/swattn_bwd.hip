@@ -840,7 +840,7 @@ __device__ __forceinline__ void dkdv_reduce(const BwdParams& p, int wg) {
   float4 acc[kUnits];
 #pragma unroll
   for (int i = 0; i < kUnits; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 2
+#pragma unroll kUnits == 1 ? 8 : 2
   for (int sp = 0; sp < sh.nch; ++sp) {
 #pragma unroll
     for (int i = 0; i < kUnits; ++i) {
@@ -1364,7 +1364,7 @@ __device__ __forceinline__ void dq_reduce(const BwdParams& p, int wg) {
   float4 acc[kUnits];
 #pragma unroll
   for (int i = 0; i < kUnits; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 2
+#pragma unroll kUnits == 1 ? 8 : 2
   for (int sp = 0; sp < nch; ++sp) {
     const int64_t piece = dq_slot_wg(p, t, sp, kvh);
 #pragma unroll

@@ -811,7 +811,8 @@ void fwd_wide_kernel(const FwdParams p) {
 // sum_c 2^LSE_c over the item's chunks (those with LSE_c = -inf skipped; a
 // row with no key in any chunk is 0 / 0 = NaN with LSE -inf, as the unsplit
 // kernel writes it).  One thread per (full item, row, 4 of the 128 d), the
-// chunks summed in order.
+// chunks summed in order.  Latency-bound.
+constexpr int kMergeAhead = 8;
 __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p) {
   const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int q4 = static_cast<int>(id & 31);
@@ -830,24 +831,42 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p) {
   if (static_cast<uint32_t>(listed) >= static_cast<uint32_t>(p.total_q)) return;
   const int qh = kvh * G + (r - slot * G);
   const int64_t ps0 = static_cast<int64_t>(fi) * p.maxc;
-  float mx = -INFINITY;
-  for (int k = 0; k < nc.x; ++k) mx = fmaxf(mx, p.part_lse[(ps0 + k) * kRowsPerItem + rr]);
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  float lsum = 0.f;
-  if (mx != -INFINITY) {
-    for (int k = 0; k < nc.x; ++k) {
-      const float lc = p.part_lse[(ps0 + k) * kRowsPerItem + rr];
-      if (lc == -INFINITY) continue;
-      const float wgt = exp2f(lc - mx);
-      const float4 o = reinterpret_cast<const float4*>(
-          p.part_o + ((ps0 + k) * kRowsPerItem + rr) * kD)[q4];
-      acc.x += wgt * o.x;
-      acc.y += wgt * o.y;
-      acc.z += wgt * o.z;
-      acc.w += wgt * o.w;
-      lsum += wgt;
+  const float* lse = p.part_lse + ps0 * kRowsPerItem + rr;
+  const float4* po = reinterpret_cast<const float4*>(p.part_o + (ps0 * kRowsPerItem + rr) * kD) + q4;
+  // The first kMergeAhead chunks' LSE and rows are loaded together, before the
+  // maximum is known.
+  float lc[kMergeAhead];
+  float4 oc[kMergeAhead];
+#pragma unroll
+  for (int k = 0; k < kMergeAhead; ++k) {
+    lc[k] = -INFINITY;
+    oc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (k < nc.x) {
+      lc[k] = lse[k * kRowsPerItem];
+      oc[k] = po[static_cast<int64_t>(k) * (kRowsPerItem * kD / 4)];
     }
   }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < kMergeAhead; ++k) mx = fmaxf(mx, lc[k]);
+#pragma unroll 4
+  for (int k = kMergeAhead; k < nc.x; ++k) mx = fmaxf(mx, lse[k * kRowsPerItem]);
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  float lsum = 0.f;
+  auto add = [&](float l, const float4& o) {
+    if (l == -INFINITY) return;   // no key in the chunk (its row is unused)
+    const float wgt = exp2f(l - mx);
+    acc.x += wgt * o.x;
+    acc.y += wgt * o.y;
+    acc.z += wgt * o.z;
+    acc.w += wgt * o.w;
+    lsum += wgt;
+  };
+#pragma unroll
+  for (int k = 0; k < kMergeAhead; ++k) add(lc[k], oc[k]);
+#pragma unroll 4
+  for (int k = kMergeAhead; k < nc.x; ++k)
+    add(lse[k * kRowsPerItem], po[static_cast<int64_t>(k) * (kRowsPerItem * kD / 4)]);
   const float inv = 1.0f / lsum;   // no key at all: 0 / 0 = NaN
   uint2 u;
   u.x = pack_bf16x2(acc.x * inv, acc.y * inv);
