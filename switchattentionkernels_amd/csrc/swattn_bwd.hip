@@ -128,7 +128,7 @@ struct BwdParams {
   int32_t count[2];          // slots per branch
   int32_t nrows[2];          // count * G
   int32_t blocks[2];         // ceil(nrows / 32)
-  int32_t items[2];          // ceil(nrows / 128)
+  int32_t items[2];          // ceil(nrows / 256)
   int64_t blk_base[2];       // packed block of (branch b, head h, block i): blk_base[b] + h * blocks[b] + i
   char* info;                // [blocks][1 KiB]
   uint16_t* zero_row;        // 128 zeros: the gather source of rows that contribute nothing
@@ -434,35 +434,41 @@ __device__ __forceinline__ void dkv_pair(const BwdParams& p, int r, int& t, int&
   }
 }
 
-// What dK/dV workgroup wg takes: share s of the row blocks of a (key tile t,
+// What a dK/dV workgroup takes: share s of the row blocks of a (key tile t,
 // KV head) pair, first .. first + nb - 1 of its n0 full and n1 local blocks
 // (from block b0lo and b1lo on).  A pair of more than dkv_chunk blocks is cut
 // into nch equal shares, at most dkv_split; shorter pairs stay whole.
-// Share 0 of every pair comes first, then share 1, ...: the shares that do not
-// exist then spread evenly over the XCDs (workgroup i runs on XCD i % 8; pair
-// by pair, an even number of slots would leave them all on the same ones).
 struct DkvShare {
-  int t, kvh, s, nch, b0lo, b1lo, n0, n1, first, nb;
+  int t, kvh, nch, b0lo, b1lo, n0, n1, first, nb;
 };
-__device__ __forceinline__ int dkv_pieces(const BwdParams& p, int n) {
-  return max(1, min(p.dkv_split, (n + p.dkv_chunk - 1) / p.dkv_chunk));
-}
-__device__ __forceinline__ DkvShare dkv_share(const BwdParams& p, int wg) {
+__device__ __forceinline__ DkvShare dkv_share(const BwdParams& p, int pair, int s) {
   DkvShare d;
-  const int pairs = p.kv_tiles_dkv * p.hkv;
-  d.s = wg / pairs;
-  dkv_pair(p, wg - d.s * pairs, d.t, d.kvh);
+  dkv_pair(p, pair, d.t, d.kvh);
   const int nt = p.kv_tiles_dkv;
   d.b0lo = p.ranges[2 * d.t];
   d.b1lo = p.ranges[2 * (nt + d.t)];
   d.n0 = max(p.ranges[2 * d.t + 1] - d.b0lo, 0);
   d.n1 = max(p.ranges[2 * (nt + d.t) + 1] - d.b1lo, 0);
   const int n = d.n0 + d.n1;
-  d.nch = dkv_pieces(p, n);
+  d.nch = max(1, min(p.dkv_split, (n + p.dkv_chunk - 1) / p.dkv_chunk));
   const int share = (n + d.nch - 1) / d.nch;
-  d.first = min(n, d.s * share);
+  d.first = min(n, s * share);
   d.nb = min(n - d.first, share);
   return d;
+}
+
+// dK/dV workgroups come in rows (tiles.h), one per share, the last share first:
+// the shares of cut pairs, then the pairs that stay whole, both by falling
+// length.  dkv_slot_wg is the inverse.
+__device__ __forceinline__ void dkv_slot(const BwdParams& p, int wg, int& pair, int& s) {
+  const int x = wg / p.hkv, kvh = wg - x * p.hkv;
+  const int row = x / p.kv_tiles_dkv;
+  s = p.dkv_split - 1 - row;
+  pair = row_entry(x - row * p.kv_tiles_dkv, row, p.kv_tiles_dkv, p.hkv) * p.hkv + kvh;
+}
+__device__ __forceinline__ int64_t dkv_slot_wg(const BwdParams& p, int pair, int s) {
+  const int tr = pair / p.hkv, kvh = pair - tr * p.hkv, row = p.dkv_split - 1 - s;
+  return (static_cast<int64_t>(row) * p.kv_tiles_dkv + row_place(tr, row, p.kv_tiles_dkv, p.hkv)) * p.hkv + kvh;
 }
 
 // The bf16 dK / dV rows of one lane's key (lane half h) from its dK^T / dV^T
@@ -496,25 +502,25 @@ __device__ __forceinline__ float4* part_unit(const BwdParams& p, int64_t wg, int
 }
 
 // dQ workgroup wg takes piece s of row tile t (full ones first) for KV head
-// kvh: piece 0 of every full tile, then piece 1, ..., then the local tiles the
-// same way, KV head fastest.  (Like the dK/dV shares, pieces that do not exist
-// spread over the XCDs.)  dq_slot_wg is the inverse.
+// kvh, KV head fastest: rows (tiles.h) of the full tiles, one per piece, the last
+// piece first, then rows of the local tiles.  Row tiles with more pieces are the
+// longer ones, so the grid runs by falling length but for the pieces' rounding.
+// dq_slot_wg is the inverse.
 __device__ __forceinline__ void dq_slot(const BwdParams& p, int wg, int& t, int& s, int& kvh) {
   kvh = wg % p.hkv;
-  const int ts = wg / p.hkv, full_slots = p.items[0] * p.dq_maxc[0];
-  if (ts < full_slots) {
-    s = ts / p.items[0];
-    t = ts - s * p.items[0];
-  } else {
-    s = (ts - full_slots) / p.items[1];
-    t = p.items[0] + ts - full_slots - s * p.items[1];
-  }
+  int x = wg / p.hkv;
+  const int full_slots = p.items[0] * p.dq_maxc[0];
+  const int b = x < full_slots ? 0 : 1;
+  x -= b ? full_slots : 0;
+  const int row = x / p.items[b];
+  s = p.dq_maxc[b] - 1 - row;
+  t = (b ? p.items[0] : 0) + row_entry(x - row * p.items[b], row, p.items[b], p.hkv);
 }
 __device__ __forceinline__ int64_t dq_slot_wg(const BwdParams& p, int t, int s, int kvh) {
-  const int64_t ts = t < p.items[0] ? static_cast<int64_t>(s) * p.items[0] + t
-                                    : static_cast<int64_t>(p.items[0]) * p.dq_maxc[0] +
-                                          static_cast<int64_t>(s) * p.items[1] + t - p.items[0];
-  return ts * p.hkv + kvh;
+  const int b = t < p.items[0] ? 0 : 1, row = p.dq_maxc[b] - 1 - s;
+  const int64_t x = static_cast<int64_t>(row) * p.items[b] +
+                    row_place(t - (b ? p.items[0] : 0), row, p.items[b], p.hkv);
+  return (x + (b ? static_cast<int64_t>(p.items[0]) * p.dq_maxc[0] : 0)) * p.hkv + kvh;
 }
 
 // Float4 unit u (= 4d + j: dQ^T block d elements 4j .. 4j+3) of (workgroup
@@ -534,8 +540,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kBwdThreads, kBwdThreads),
   // stages, its source pointer) then stay scalar selects.
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
-  const DkvShare sh = dkv_share(p, blockIdx.x);
-  if (sh.s >= sh.nch) return;
+  int pair, share;
+  dkv_slot(p, blockIdx.x, pair, share);
+  const DkvShare sh = dkv_share(p, pair, share);
+  if (share >= sh.nch) return;
   const int t = sh.t, kvh = sh.kvh;
   const int kw0 = t * kKeysDkv + 32 * wave;   // this wave's first key
   const int key = kw0 + n;                    // this lane's key (B column)
@@ -724,8 +732,10 @@ __device__ __forceinline__ void dkdv_wide(const BwdParams& p, char* smem, int wg
   const int j = lane & 31, hh = lane >> 5;
   // The pair's blocks run in the loop's order; a share of a cut pair leaves
   // fp32 partials.
-  const DkvShare sh = dkv_share(p, wg);
-  if (sh.s >= sh.nch) return;   // uniform
+  int pair, share;
+  dkv_slot(p, wg, pair, share);
+  const DkvShare sh = dkv_share(p, pair, share);
+  if (share >= sh.nch) return;   // uniform
   const int t = sh.t, kvh = sh.kvh, b0lo = sh.b0lo, b1lo = sh.b1lo, n0 = sh.n0;
   const int first = sh.first, nb = sh.nb;
   const bool split = sh.nch > 1;
@@ -828,10 +838,9 @@ template <int kUnits>
 __device__ __forceinline__ void dkdv_reduce(const BwdParams& p, int wg) {
   constexpr int kWgs = kDkvReduceWgs / kUnits;
   const int pair = wg / kWgs;
-  const DkvShare sh = dkv_share(p, pair);
+  const DkvShare sh = dkv_share(p, pair, 0);
   if (sh.nch <= 1) return;   // stored whole by its workgroup
   const int kvh = sh.kvh;
-  const int64_t pairs = static_cast<int64_t>(p.kv_tiles_dkv) * p.hkv;
   const int lane = threadIdx.x & 63;
   // Unit i of the thread: id = (pair-relative workgroup, i, thread).
   const int id0 = (wg - pair * kWgs) * kUnits * kThreads + threadIdx.x;
@@ -845,7 +854,7 @@ __device__ __forceinline__ void dkdv_reduce(const BwdParams& p, int wg) {
 #pragma unroll
     for (int i = 0; i < kUnits; ++i) {
       const int id = id0 + i * kThreads;
-      const float4 a = *part_unit(p, sp * pairs + pair, wave_of(id), unit(id), lane);
+      const float4 a = *part_unit(p, dkv_slot_wg(p, pair, sp), wave_of(id), unit(id), lane);
       acc[i].x += a.x;
       acc[i].y += a.y;
       acc[i].z += a.z;

@@ -56,6 +56,28 @@ __device__ __forceinline__ int wave_max(int x) {
   for (int off = 32; off >= 1; off >>= 1) x = max(x, __shfl_xor(x, off));
   return x;
 }
+// Work cut into several parts per entry (tile) is laid out in rows of workgroups,
+// one row per part with all n entries in order, KV head fastest in an entry.
+// Entries of few parts leave gaps in most rows and the long entries stand wherever
+// the sequences end, so that each row starts one entry later on the XCDs than the
+// row before (workgroup i runs on XCD i % 8): neither the gaps nor a period in the
+// long ones then collects on a few XCDs.  Rows of a multiple of 8 KV heads put a
+// head's parts on one XCD, all of them alike, and are not turned.  row_entry: the
+// entry at place x of a row; row_place: its inverse.
+__device__ __forceinline__ int row_turn(int row, int n, int hkv) {
+  const uint32_t period = 8u >> min(__builtin_ctz(hkv), 3);   // entries after which a row meets the same XCDs
+  return static_cast<int>((static_cast<uint32_t>(row) * (1u - static_cast<uint32_t>(n))) & (period - 1u));
+}
+__device__ __forceinline__ int row_entry(int x, int row, int n, int hkv) {
+  int e = x - row_turn(row, n, hkv);
+  while (e < 0) e += n;
+  return e;
+}
+__device__ __forceinline__ int row_place(int entry, int row, int n, int hkv) {
+  int x = entry + row_turn(row, n, hkv);
+  while (x >= n) x -= n;
+  return x;
+}
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   const __bf16 ha = static_cast<__bf16>(a), hb = static_cast<__bf16>(b);
   return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, ha)) |
