@@ -101,7 +101,7 @@ constexpr size_t kPartBytesPerWg = static_cast<size_t>(kBwdWaves) * kPartUnits *
 // tile, KV head) pairs over their row blocks.
 constexpr int64_t kDkvTargetWgs = 512;
 constexpr int kDkvMaxSplit = 16;
-constexpr int64_t kDkvMinBlocks = 4;   // row blocks a cut pair's share takes at least
+constexpr int kDkvMinBlocks = 4;   // row blocks a cut pair's share takes at least
 // dQ workgroups that run at once (one per CU: the 96 KiB ring allows one).
 constexpr int64_t kDqSlots = 256;
 // dQ piece partials: per workgroup and wave, 16 float4 units per lane (dQ^T
@@ -135,7 +135,7 @@ struct BwdParams {
   int32_t* ranges;           // [2][kv_tiles_dkv][2] block ranges
   float* dkv_part;           // dK/dV split partials (dkv_split > 1): [workgroup][8 waves][32][64 lanes] float4
   int32_t dkv_split;         // dK/dV workgroup slots per (key tile, KV head)
-  int32_t dkv_chunk;         // row blocks per dK/dV workgroup (a pair is cut into at most dkv_split)
+  int32_t dkv_jobs;          // dK/dV pairs + dQ row tiles, over all KV heads (dkv_chunk)
   int32_t dkv_wgs;           // bwd_wide_kernel: workgroups below this are dK/dV's, the rest dQ's
   int32_t prep_wgs;          // bwd_prep_kernel: workgroups below this prepare blocks, the rest ranges
   int32_t dkv_batches;       // > 1: key tiles ordered tile-in-sequence-major over this many sequences
@@ -434,6 +434,37 @@ __device__ __forceinline__ void dkv_pair(const BwdParams& p, int r, int& t, int&
   }
 }
 
+// The row blocks c a dK/dV workgroup may take: as many as the grid has time per
+// CU.  Both products run in one grid (bwd_wide_kernel), so a pair is too long
+// only against all of it; cutting finer starts more workgroups and writes and
+// reads back 256 KiB of partials for each.  In tenths of a us: a row block takes
+// 16, a dQ key tile 22 (a row tile has about one per two of its blocks' key
+// tiles), a workgroup's start and end 150, and a share of a cut pair 225 more, so
+//   16 c + 150 = per_cu + 225 (blocks / c) / CUs,
+// per_cu being the time per CU of the uncut grid.  (150 shapes of up to 4000
+// positions and 110 of up to 16384, backward, mean over the best of each: 0.8 and
+// 1.3 % with this, 3.4 and 3.2 % without the last term; the finest cut is 5 %
+// slower.)  The blocks are counted from the ranges: the host knows neither where
+// packed sequences end nor which positions are full.  (Taken from the list
+// lengths alone, 64 packed sequences of 128 keys and one of 8192, Hq8/Hkv2, took
+// 358 us, counted 234; eight of 300 to 1400 keys, Hq64/Hkv8, every row full, 550
+// and 263 us.)  The grid and the reduce must find the same value: no contraction,
+// and one float sum in one order.
+__device__ __forceinline__ float dkv_chunk(const BwdParams& p) {
+#pragma clang fp contract(off)
+  const int lane = count_below(~uint64_t{0});
+  const int2* ranges = reinterpret_cast<const int2*>(p.ranges);
+  float blocks = 0.f;
+  for (int i = lane; i < 2 * p.kv_tiles_dkv; i += 64) {
+    const int2 r = ranges[i];
+    blocks += static_cast<float>(max(r.y - r.x, 0));
+  }
+  blocks = wave_sum(blocks) * p.hkv;
+  const float b = (27.f * blocks + 150.f * p.dkv_jobs) * (1.f / kDqSlots) - 150.f;
+  const float c = (b + __builtin_amdgcn_sqrtf(b * b + (64.f * 225.f / kDqSlots) * blocks)) * (1.f / 32);
+  return max(c, static_cast<float>(kDkvMinBlocks));
+}
+
 // What a dK/dV workgroup takes: share s of the row blocks of a (key tile t,
 // KV head) pair, first .. first + nb - 1 of its n0 full and n1 local blocks
 // (from block b0lo and b1lo on).  A pair of more than dkv_chunk blocks is cut
@@ -450,7 +481,11 @@ __device__ __forceinline__ DkvShare dkv_share(const BwdParams& p, int pair, int 
   d.n0 = max(p.ranges[2 * d.t + 1] - d.b0lo, 0);
   d.n1 = max(p.ranges[2 * (nt + d.t) + 1] - d.b1lo, 0);
   const int n = d.n0 + d.n1;
-  d.nch = max(1, min(p.dkv_split, (n + p.dkv_chunk - 1) / p.dkv_chunk));
+  d.nch = 1;
+  if (p.dkv_split > 1) {   // (uniform) 512 pairs or more are never cut
+    const float shares = ceilf(n * __builtin_amdgcn_rcpf(dkv_chunk(p)));
+    d.nch = __builtin_amdgcn_readfirstlane(max(1, static_cast<int>(min(shares, static_cast<float>(p.dkv_split)))));
+  }
   const int share = (n + d.nch - 1) / d.nch;
   d.first = min(n, s * share);
   d.nb = min(n - d.first, share);
@@ -1430,7 +1465,7 @@ __global__ __launch_bounds__(kThreads) void bwd_reduce_kernel(const BwdParams p)
 constexpr int64_t kReduceWide = 4096;
 
 struct BwdLayout {
-  int64_t blocks[2], items[2], total_blocks, kv_tiles_dkv, dkv_split, dkv_chunk, dq_chunk, dq_maxc[2];
+  int64_t blocks[2], items[2], total_blocks, kv_tiles_dkv, dkv_split, dkv_jobs, dq_chunk, dq_maxc[2];
   size_t off_info, off_zero, off_ranges, off_part, off_dq_nch, off_dq_part, bytes;
 };
 
@@ -1475,8 +1510,8 @@ inline BwdLayout bwd_layout(int64_t seq_kv, int64_t total_kv, int32_t heads_kv, 
   L.kv_tiles_dkv = ceil_div(total_kv, kKeysDkv);
   // Fewer (key tile, KV head) pairs than two rounds of workgroups: room to cut
   // each pair over its row blocks, so that the longest pair (the first key
-  // tile sees every full row) does not set the grid's length (dkv_chunk below
-  // says which pairs are cut).
+  // tile sees every full row) does not set the grid's length (dkv_chunk says
+  // which pairs are cut).
   const int64_t pairs = L.kv_tiles_dkv * heads_kv;
   L.dkv_split = pairs >= kDkvTargetWgs ? 1
                 : std::min<int64_t>(kDkvMaxSplit, ceil_div(kDkvTargetWgs, pairs));
@@ -1524,21 +1559,7 @@ inline BwdLayout bwd_layout(int64_t seq_kv, int64_t total_kv, int32_t heads_kv, 
     o += static_cast<size_t>(heads_kv * slots) * kDqPartBytesPerWg;
   }
   L.bytes = o;
-
-  // Within that room, the row blocks a dK/dV workgroup may take: as many as
-  // the grid has time per CU.  Both products run in one grid
-  // (bwd_wide_kernel), so a pair is too long only against all of it; cutting
-  // finer writes and reads back 256 KiB of partials more per workgroup.  (Times
-  // in tenths of a us: a row block 16, a dQ key tile 22, starting and ending a
-  // workgroup 150.  Shares of 1/2, 3/4 and 1 of the time per CU, forward and
-  // backward on the GPU: B1 S2048 Hq32/Hkv8 W512 192, 173 and 159 us; B1
-  // S16384 Hq4/Hkv1 W1024 477, 464 and 456; B2 S4096 Hq32/Hkv8 774, 732, 732;
-  // 5/4 of it would leave the last of two rounds half empty.)
-  const int64_t full_kt = ceil_div(seq_kv, kKeysDkv);
-  const int64_t local_kt = std::min<int64_t>(full_kt, ceil_div(window, kKeysDkv) + 1);
-  const int64_t dkv = heads_kv * (L.blocks[0] * (full_kt + 1) / 2 + L.blocks[1] * local_kt);
-  const int64_t per_cu = (16 * dkv + 150 * pairs + 22 * est + 150 * q_items) / kDqSlots;
-  L.dkv_chunk = std::min<int64_t>(INT32_MAX / 2, std::max<int64_t>(kDkvMinBlocks, (per_cu - 150) / 16));
+  L.dkv_jobs = pairs + q_items;
   return L;
 }
 
@@ -1650,7 +1671,7 @@ extern "C" int swattn_prefill_bwd(const void* q, const void* k, const void* v, c
   p.total_kv = static_cast<int32_t>(total_kv);
   p.kv_tiles_dkv = static_cast<int32_t>(L.kv_tiles_dkv);
   p.dkv_split = static_cast<int32_t>(L.dkv_split);
-  p.dkv_chunk = static_cast<int32_t>(L.dkv_chunk);
+  p.dkv_jobs = static_cast<int32_t>(std::min<int64_t>(INT32_MAX, L.dkv_jobs));
   // Several sequences that each hold whole 256-key tiles: interleave them.
   p.dkv_batches = (batch > 1 && seq_kv % kKeysDkv == 0) ? batch : 1;
   p.dkv_part = reinterpret_cast<float*>(ws + L.off_part);

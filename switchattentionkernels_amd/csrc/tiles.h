@@ -46,6 +46,17 @@ __device__ __forceinline__ float xor32_sum(float x) {
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// Sum over the wave, the same in every lane: DPP moves within 16 lanes, then
+// lane swaps (no LDS round trips).
+__device__ __forceinline__ float wave_sum(float x) {
+  constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kHalfMirror = 0x141, kMirror = 0x140;
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kXor1, 0xf, 0xf, false));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kXor2, 0xf, 0xf, false));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kHalfMirror, 0xf, 0xf, false));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kMirror, 0xf, 0xf, false));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return xor32_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
 __device__ __forceinline__ int wave_min(int x) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) x = min(x, __shfl_xor(x, off));

@@ -82,3 +82,59 @@ def test_shares_of_recurring_long_pairs_spread_over_the_xcds():
     assert int(per_xcd.max()) <= 1.5 * int(shares.sum()) / 8
 
 
+def _rows_blocks(cu, group, tiles):
+    """Row blocks that see each 256-key tile, every row full: 32-row blocks of
+    the rows whose range [sequence start, position] overlaps the tile."""
+    rows = [(a, p) for a, e in zip(cu, cu[1:]) for p in range(a, e)]
+    out = []
+    for t in range(tiles):
+        seen = [p for a, p in rows if p >= 256 * t and a < 256 * (t + 1)]
+        out.append(-(-(seen[-1] + 1) * group // 32) - seen[0] * group // 32)
+    return out
+
+
+def test_packed_sequences_are_cut_by_what_their_tiles_see():
+    """Eight short sequences, every row full: a tile is seen by its own
+    sequence's rows only, many fewer than the list lengths allow for.  A
+    pair that takes longer than the grid's time per CU must be cut, and the
+    gradients are those of the sequences one by one."""
+    cu = [0, 300, 700, 1000, 1300, 1500, 1800, 2143, 3564]
+    s, hq, hkv, w = cu[-1], 64, 8, 473
+    problem = _problem(1, s, hq, hkv, torch.ones(1, s, dtype=torch.bool), w, cu=cu)
+    grads, shares = _backward(problem, w)
+    n = _rows_blocks(cu, hq // hkv, shares.shape[1] // hkv)
+    per_cu = 2.7 * hkv * sum(n) / 256   # us: a row block 1.6, its part of dQ 1.1
+    cut = shares.sum(0).view(-1, hkv)   # (8 KV heads: every row holds the pairs in order)
+    print("[cut] blocks", n, "time per CU", round(per_cu), "shares", cut[:, 0].tolist(), flush=True)
+    for tile, blocks in enumerate(n):
+        if 1.6 * blocks > 2 * per_cu:
+            assert int(cut[tile].min()) >= 2, (tile, blocks)
+        if 1.6 * blocks < 0.5 * per_cu:
+            assert int(cut[tile].max()) == 0, (tile, blocks)
+    assert int(cut.max()) >= 2
+    q, k, v, do, o, lse = problem[:6]
+    for a, e in zip(cu, cu[1:]):
+        full, local = build_switch_query_indices(torch.ones(1, e - a, dtype=torch.bool, device=DEV))
+        one = [t[:, a:e].contiguous() for t in (q, k, v, o, lse, do)]
+        ref = switch_gqa_prefill_backward(*one, full, local, window_size=w)
+        for name, got, want in zip(("dq", "dk", "dv"), grads, ref):
+            g, r = got[:, a:e].float(), want.float()
+            assert float((g - r).norm() / r.norm()) <= 2e-3, (name, a)
+
+
+@pytest.mark.parametrize("b,s,hq,hkv,w,p", [
+    (2, 2048, 8, 4, 256, 0.9),      # whole 256-key tiles of two sequences, few shares
+    (2, 1792, 16, 2, 200, 0.25),
+    (3, 1000, 8, 2, 300, 0.5)])     # tiles that straddle the sequences
+def test_cut_pairs_of_several_sequences(b, s, hq, hkv, w, p):
+    gen = torch.Generator().manual_seed(b * s)
+    mask = torch.rand(b, s, generator=gen) < p
+    problem = _problem(b, s, hq, hkv, mask, w)
+    grads, shares = _backward(problem, w)
+    per_slot = shares.sum(1).tolist()
+    print(f"[cut] B{b} S{s} shares per slot, last slot first", per_slot, flush=True)
+    assert per_slot[-1] > 0 and per_slot == sorted(per_slot)   # some cut, few of them finely
+    assert per_slot[0] < shares.shape[1]
+    q, k, v, do = (t.cpu() for t in problem[:4])
+    for got, ref, name in zip(grads, _oracle(q, k, v, do, mask, w), ("dq", "dk", "dv")):
+        _grad_close(got, ref, f"cut b{b} s{s} {name}")
