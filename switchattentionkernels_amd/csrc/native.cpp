@@ -37,12 +37,17 @@ const int32_t* i32(const optional<Tensor>& t) { return t.has_value() ? i32(*t) :
 
 // Pinned host memory for a compaction's counts.  One buffer per thread: a call
 // waits for its counts before it returns, so that a thread has at most one
-// compaction in flight.
+// compaction in flight.  After a HIP error a kernel may still be queued that
+// reports there: the buffer is then left to it for good.
+thread_local c10::DataPtr t_words;
 int32_t* host_words() {
-  thread_local c10::DataPtr buf;
-  if (!buf)
-    buf = at::getHostAllocator(at::kCUDA)->allocate(SWATTN_COMPACT_HOST_WORDS * sizeof(int32_t));
-  return static_cast<int32_t*>(buf.get());
+  if (!t_words)
+    t_words = at::getHostAllocator(at::kCUDA)->allocate(SWATTN_COMPACT_HOST_WORDS * sizeof(int32_t));
+  return static_cast<int32_t*>(t_words.get());
+}
+void abandon_host_words() {
+  (void)t_words.release_context();
+  t_words = c10::DataPtr();
 }
 
 // (full, local) of a byte mask (dtype -1) or of router logits.
@@ -62,6 +67,7 @@ std::tuple<Tensor, Tensor> compact(const Tensor& x, int64_t dtype, double thresh
                                  ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
                                  as_stream(stream));
   }
+  if (status > 0) abandon_host_words();
   check(status, dtype < 0 ? "swattn_compact" : "swattn_compact_logits");
   const int64_t nf = host[0];
   return {out.narrow(0, 0, nf), out.narrow(0, nf, n - nf)};

@@ -474,7 +474,12 @@ int swattn_compact_wait(const void* x, int32_t dtype, int64_t n, float threshold
                                host, workspace, workspace_bytes, stream, name, &blocks)
                 : compact_logits_impl(x, dtype, n, threshold, indices, host, workspace,
                                       workspace_bytes, stream, name, &blocks);
-  if (status != SWATTN_OK) return status;
+  if (status != SWATTN_OK) {
+    // A HIP error, perhaps one that an earlier call left pending: the kernel may
+    // be queued all the same, and must not report into the next call's words.
+    if (status > 0) (void)hipStreamSynchronize(as_stream(stream));
+    return status;
+  }
   // Poll the blocks' words for a while; then, or where none report, wait for
   // the stream (it may hold any amount of earlier work, or have failed).
   volatile int32_t* word = host + 2;

@@ -15,7 +15,9 @@ extern "C" {
  * and host[1] hold the counts.
  *   host  SWATTN_COMPACT_HOST_WORDS int32 of pinned host memory, one call at a
  *         time.  The kernel reports there; a device copy of the counts and a
- *         stream synchronisation would take about 8 us more.
+ *         stream synchronisation would take about 8 us more.  After a HIP error
+ *         (a positive status) the stream was synchronised if it could be; if not,
+ *         a kernel may report later, so that host is not to be used again.
  */
 #define SWATTN_COMPACT_HOST_WORDS 66
 int swattn_compact_wait(const void* x, int32_t dtype, int64_t n, float threshold, int32_t* indices,
