@@ -467,6 +467,10 @@ int swattn_compact_wait(const void* x, int32_t dtype, int64_t n, float threshold
                         int32_t* host, void* workspace, size_t workspace_bytes, void* stream) {
   const char* name = dtype < 0 ? "swattn_compact" : "swattn_compact_logits";
   if (host == nullptr) return invalid(std::string(name) + ": null pointer");
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(as_stream(stream), &capture) == hipSuccess &&
+      capture != hipStreamCaptureStatusNone)   // before a launch that nothing could wait for
+    return invalid(std::string(name) + ": waits for its result and cannot be captured");
   for (int i = 0; i < SWATTN_COMPACT_HOST_WORDS; ++i) host[i] = 0;
   int blocks = 0;
   const int status =

@@ -18,6 +18,7 @@ extern "C" {
  *         stream synchronisation would take about 8 us more.  After a HIP error
  *         (a positive status) the stream was synchronised if it could be; if not,
  *         a kernel may report later, so that host is not to be used again.
+ * A stream under capture is refused (SWATTN_EINVAL) before anything is launched.
  */
 #define SWATTN_COMPACT_HOST_WORDS 66
 int swattn_compact_wait(const void* x, int32_t dtype, int64_t n, float threshold, int32_t* indices,

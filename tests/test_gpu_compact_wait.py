@@ -132,3 +132,23 @@ def test_failed_call_leaves_the_next_alone(n):
         else:
             assert torch.equal(full.cpu(), want[0]) and torch.equal(local.cpu(), want[1])
     assert not wrong, (want[0].numel(), wrong)
+
+
+@pytest.mark.parametrize("n", [0, 5000, 300000])
+def test_capture_is_refused(n):
+    """A call under capture raises and leaves the capture as it was."""
+    mask = _mask(3, n)
+    dev = mask.to(DEV)
+    x = torch.zeros(8, device=DEV)
+    build_switch_query_indices(dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        with pytest.raises(RuntimeError, match="captur"):
+            build_switch_query_indices(dev)
+    for _ in range(3):
+        graph.replay()
+    full, local = build_switch_query_indices(dev)
+    want = _expect(mask)
+    assert torch.equal(full.cpu(), want[0]) and torch.equal(local.cpu(), want[1])
+    assert x.tolist() == [3.0] * 8
