@@ -387,17 +387,20 @@ __global__ __launch_bounds__(256) void metadata_args_kernel(const CuArgs cu, int
 
 // Whether each list's key bounds are non-decreasing along it (a start past its
 // row's end counts as the end): what the backward's searches need.  One thread
-// per neighbouring pair of both lists; a listed position outside [0, total_q)
-// is never dereferenced and fails the check.
+// per entry of both lists and its successor; a listed position outside
+// [0, total_q) is never dereferenced and fails the check.
 __global__ __launch_bounds__(256) void check_bounds_kernel(
     const int32_t* __restrict__ full, int64_t nf, const int32_t* __restrict__ local, int64_t nl,
     const int32_t* __restrict__ full_starts, const int32_t* __restrict__ local_starts,
     const int32_t* __restrict__ ends, int64_t total_q, int32_t* __restrict__ flags) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   auto falls = [&](const int32_t* list, int64_t n, const int32_t* starts) {
+    if (i >= n) return false;
+    const int32_t a = list[i];
+    if (a < 0 || a >= total_q) return true;
     if (i + 1 >= n) return false;
-    const int32_t a = list[i], b = list[i + 1];
-    if (a < 0 || a >= total_q || b < 0 || b >= total_q) return true;
+    const int32_t b = list[i + 1];
+    if (b < 0 || b >= total_q) return true;
     const int32_t ea = ends[a], eb = ends[b];
     return eb < ea || min(starts[b], eb) < min(starts[a], ea);
   };
@@ -565,7 +568,7 @@ int swattn_check_bounds(const int32_t* full, int64_t n_full, const int32_t* loca
   const hipStream_t st = as_stream(stream);
   hipLaunchKernelGGL(flags_clear_kernel, dim3(1), dim3(1), 0, st, flags);
   const int64_t n = n_full > n_local ? n_full : n_local;
-  if (n > 1)
+  if (n > 0)
     hipLaunchKernelGGL(check_bounds_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, st, full, n_full,
                        local, n_local, full_starts, local_starts, causal_ends, total_q, flags);
   return launch_status("swattn_check_bounds");

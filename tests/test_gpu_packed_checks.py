@@ -40,7 +40,7 @@ def test_metadata_sequence_counts(nseq, same):
 @pytest.mark.parametrize("nf,nl,fault", [
     (0, 1, None), (1, 0, None), (257, 300, None), (64, 65, "full_end"), (1000, 513, "full_start"),
     (2, 256, "local_start"), (256, 2, "local_end"), (300, 300, "empty_start"),
-    (300, 300, "range")])
+    (300, 300, "range"), (0, 1, "range"), (1, 1, "range"), (300, 1, "range")])
 def test_check_bounds(nf, nl, fault):
     n = nf + nl
     gen = torch.Generator().manual_seed(n)
