@@ -48,6 +48,8 @@ SIGNATURES = {
 
 # Entry points of libswattn.so for this package only (csrc/swattn_internal.h).
 INTERNAL_SIGNATURES = {
+    "swattn_compact_wait": (ctypes.c_int, [_vp, _i32, _i64, ctypes.c_float, _vp, _vp, _vp,
+                                           ctypes.c_size_t, _vp]),
     "swattn_build_metadata_host": (ctypes.c_int, [_vp, _vp, _i32, _i64, _i64, _i32,
                                                   _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "swattn_check_bounds": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp]),

@@ -605,11 +605,11 @@ int swattn_build_metadata_host(const int32_t* cu_seqlens_q, const int32_t* cu_se
   if (st != SWATTN_OK) return st;
   if (num_seqs > SWATTN_METADATA_HOST_MAX_SEQS)
     return invalid("swattn_build_metadata_host: too many sequences (use swattn_build_metadata)");
-  const int64_t n = total_q > total_kv ? total_q : total_kv;
-  if (n == 0) return SWATTN_OK;
   CuArgs cu{};
   memcpy(cu.q, cu_seqlens_q, (num_seqs + 1) * sizeof(int32_t));
   memcpy(cu.kv, cu_seqlens_kv, (num_seqs + 1) * sizeof(int32_t));
+  const int64_t n = total_q > total_kv ? total_q : total_kv;
+  if (n == 0) return SWATTN_OK;
   hipLaunchKernelGGL(metadata_args_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, as_stream(stream),
                      cu, num_seqs, total_q, total_kv, window, o);
   return launch_status(name);

@@ -25,7 +25,7 @@ CHILD = textwrap.dedent('''
     spec = importlib.util.spec_from_file_location("abi", sys.argv[1])
     abi = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(abi)
-    L = abi.bind(ctypes.CDLL(sys.argv[2]))
+    L = abi.bind(abi.bind(ctypes.CDLL(sys.argv[2])), abi.INTERNAL_SIGNATURES)
     P = 0x10000   # placeholder address: every call below returns before using it
     EINVAL, EWS = -1, -2
 
@@ -123,6 +123,37 @@ CHILD = textwrap.dedent('''
     ws_unaligned(L.swattn_decode_fwd(P, P, P, P, P, P, P, 4, 100, 8, 2, 128, 64, 0.1, W, 1 << 30,
                                      None), "swattn_decode_fwd")
     ws_unaligned(L.swattn_compact(P, 100000, P, P, W, 1 << 20, None), "swattn_compact")
+    # entry points of the package's own layer
+    words = (ctypes.c_int32 * 66)()
+    err(L.swattn_compact_wait(P, -1, 10, 0.0, P, None, P, 1 << 20, None), EINVAL, "swattn_compact")
+    err(L.swattn_compact_wait(None, -1, 10, 0.0, P, words, P, 1 << 20, None), EINVAL,
+        "swattn_compact")
+    err(L.swattn_compact_wait(P, -1, -1, 0.0, P, words, P, 1 << 20, None), EINVAL,
+        "swattn_compact")
+    err(L.swattn_compact_wait(P, 7, 10, 0.0, P, words, P, 1 << 20, None), EINVAL,
+        "swattn_compact_logits")
+    err(L.swattn_compact_wait(P, 0, 100000, 0.0, P, words, None, 0, None), EWS,
+        "swattn_compact_logits")
+    assert list(words) == [0] * 66
+    n = 257
+    offsets = (ctypes.c_int32 * n)(*range(n))   # those of 256 sequences, no more
+    host = lambda cq, ck, num, tq, w, out: L.swattn_build_metadata_host(
+        cq, ck, num, tq, tq, w, out, P, P, P, P, P, P, None)
+    err(host(offsets, offsets, n, n, 4, P), EINVAL, "swattn_build_metadata_host")
+    assert b"too many sequences" in L.swattn_last_error()
+    err(host(offsets, None, 2, 2, 4, P), EINVAL, "swattn_build_metadata_host")
+    err(host(offsets, offsets, 2, 2, 0, P), EINVAL, "swattn_build_metadata_host")
+    err(host(offsets, offsets, 0, 2, 4, P), EINVAL, "swattn_build_metadata_host")
+    err(host(offsets, offsets, 2, 2, 4, None), EINVAL, "swattn_build_metadata_host")
+    # Nothing to write: the offsets are copied, and no launch follows.
+    assert host(offsets, offsets, 256, 0, 4, None) == 0
+    bounds = lambda nf, full, starts, ends, flags: L.swattn_check_bounds(
+        full, nf, P, 3, starts, P, ends, 10, flags, None)
+    err(bounds(-1, P, P, P, P), EINVAL, "swattn_check_bounds")
+    err(bounds(5, None, P, P, P), EINVAL, "swattn_check_bounds")
+    err(bounds(5, P, None, P, P), EINVAL, "swattn_check_bounds")
+    err(bounds(5, P, P, None, P), EINVAL, "swattn_check_bounds")
+    err(bounds(5, P, P, P, None), EINVAL, "swattn_check_bounds")
     print("host checks ok")
 ''')
 
