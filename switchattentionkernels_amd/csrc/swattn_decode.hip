@@ -49,9 +49,8 @@ struct DecodeParams {
   float* part_o;     // [slot][G][128] unnormalised sum of p * v, per workgroup and pair
   float* part_ml;    // [slot][G][2]   maximum (exp2 domain) and sum of p
   int32_t* list;     // sequences with keys, in order                      (plan kernel)
-  uint4* plan;       // [0] {positions per workgroup, positions of the line}; [1 + b] {position of
-                     // sequence b's first key, its keys, its rank among those with keys,
-                     // positions per pair}
+  uint4* plan;       // [0] {positions per workgroup, positions of the line (low, high)}; [1 + b]
+                     // plan_entry of sequence b
   uint16_t* out;
   float* lse;
   int cache_len;     // L
@@ -83,9 +82,10 @@ __device__ __forceinline__ void key_range(const DecodeParams& p, int b, int& lo,
 }
 
 // The line's layout, chosen from the total of routed keys and the number of
-// pairs that have any (both over all KV heads).  Positions and lengths are
-// 32-bit: the line holds at most one entry per row of the K cache, and a cache
-// of 2^31 rows of 256 bytes fits no device (the host refuses it).
+// pairs that have any (both over all KV heads).  Positions are 32-bit where the
+// workgroups plan for themselves, which they do for caches of fewer than 2^31
+// rows (512 GiB), and 64-bit in the plan kernel; a share and a pair's keys fit 32
+// bits in both (the host sees to it).
 //
 // * Shared: every pair takes its keys plus p.pad positions (what starting a
 //   pair costs, in keys), and the line is cut into p.target equal shares,
@@ -104,25 +104,28 @@ __device__ __forceinline__ void key_range(const DecodeParams& p, int b, int& lo,
 //
 // A share is at least kMinShare keys and at least ceil(L / 255), so that a
 // pair is spread over at most 256 workgroups, rounded up to 16.
+template <typename Pos>
 struct Line {
-  uint32_t share, total, aligned;   // total: positions of the line
+  uint32_t share, aligned;
+  Pos total;   // positions of the line
   __device__ __forceinline__ uint32_t length(uint32_t n, uint32_t pad) const {
     return n == 0 ? 0u : aligned ? (n + share - 1u) / share * share : n + pad;
   }
 };
-__device__ __forceinline__ Line plan_line(const DecodeParams& p, uint32_t keys, uint32_t pairs) {
+template <typename Pos>
+__device__ __forceinline__ Line<Pos> plan_line(const DecodeParams& p, Pos keys, uint32_t pairs) {
   const uint32_t target = p.target;
   const uint32_t by_len = (static_cast<uint32_t>(p.cache_len) + kMaxSplitsDev - 2u) / (kMaxSplitsDev - 1u);
   const uint32_t least = max(by_len, static_cast<uint32_t>(kMinShare));
-  Line L;
+  Line<Pos> L;
   L.total = keys + pairs * p.pad;
-  L.share = (L.total + target - 1u) / target;
+  L.share = static_cast<uint32_t>((L.total + target - 1u) / target);
   L.aligned = 0u;
   if (pairs < target) {
-    const uint32_t a = max((keys + target - pairs - 1u) / (target - pairs), least);
+    const Pos a = max((keys + target - pairs - 1u) / (target - pairs), static_cast<Pos>(least));
     if (a <= max(L.share, least) + kAlignSlack) {
       L.aligned = 1u;
-      L.share = a;
+      L.share = static_cast<uint32_t>(a);
     }
   }
   if (L.aligned == 0u && L.share >= kLongShare) L.share = (L.share + 1u) / 2u;
@@ -132,18 +135,20 @@ __device__ __forceinline__ Line plan_line(const DecodeParams& p, uint32_t keys, 
 
 // Exclusive prefix sums over the workgroup's threads of (keys, cnt), and both
 // totals; one barrier.  (kUse: calls of one kernel use separate LDS words.)
-template <int kWaves, int kUse>
-__device__ __forceinline__ void scan_keys(uint32_t keys, uint32_t cnt, uint32_t& keys_before,
-                                          uint32_t& cnt_before, uint32_t& keys_total,
+template <int kWaves, int kUse, typename Pos>
+__device__ __forceinline__ void scan_keys(Pos keys, uint32_t cnt, Pos& keys_before,
+                                          uint32_t& cnt_before, Pos& keys_total,
                                           uint32_t& cnt_total) {
-  __shared__ uint32_t s_keys[kWaves], s_cnt[kWaves];
+  __shared__ Pos s_keys[kWaves];
+  __shared__ uint32_t s_cnt[kWaves];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t ik = keys, ic = cnt;
+  Pos ik = keys;
+  uint32_t ic = cnt;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t uk = __shfl_up(ik, off);
+    const Pos uk = __shfl_up(ik, off);
     const uint32_t uc = __shfl_up(ic, off);
-    ik += lane >= off ? uk : 0u;
+    ik += lane >= off ? uk : Pos{0};
     ic += lane >= off ? uc : 0u;
   }
   if (lane == 63) {
@@ -153,20 +158,41 @@ __device__ __forceinline__ void scan_keys(uint32_t keys, uint32_t cnt, uint32_t&
   __syncthreads();
   keys_before = ik - keys;
   cnt_before = ic - cnt;
-  keys_total = cnt_total = 0u;
+  keys_total = Pos{0};
+  cnt_total = 0u;
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) {
-    keys_before += w < wave ? s_keys[w] : 0u;
+    keys_before += w < wave ? s_keys[w] : Pos{0};
     cnt_before += w < wave ? s_cnt[w] : 0u;
     keys_total += s_keys[w];
     cnt_total += s_cnt[w];
   }
 }
 
+// Sequence b's place on the line as the merge (and the listed plan) reads it:
+// position of its first key, its keys, its rank among those with keys, positions
+// per pair.  Ranks are below 65536, so the position has 48 bits.
+struct SeqPlace {
+  uint64_t off;
+  uint32_t n, rank, len;
+};
+__device__ __forceinline__ uint4 plan_entry(uint64_t off, uint32_t n, uint32_t rank, uint32_t len) {
+  return make_uint4(static_cast<uint32_t>(off), n, rank | static_cast<uint32_t>(off >> 32) << 16, len);
+}
+__device__ __forceinline__ SeqPlace seq_place(const uint4& e) {
+  return SeqPlace{e.x | static_cast<uint64_t>(e.z >> 16) << 32, e.y, e.z & 0xffffu, e.w};
+}
+
+// a / b where the quotient fits 32 bits.
+__device__ __forceinline__ uint32_t quotient(uint64_t a, uint32_t b) {
+  return (a >> 32) == 0 ? static_cast<uint32_t>(a) / b : static_cast<uint32_t>(a / b);
+}
+
 // A sequence with keys: its index, first key, number of keys, and the
 // positions each of its pairs takes on the line.
 struct SeqEntry {
-  int b, lo, n, len;
+  int b, lo, n;
+  uint32_t len;
 };
 
 // Where a split workgroup starts on the line: position `key` of pair (entry r,
@@ -175,13 +201,13 @@ struct SplitStart {
   uint32_t r, kvh, key, take;
 };
 
-// Start at `pos` of the line inside the sequence of rank r, whose pairs take
-// len positions each from `off` on.
-__device__ __forceinline__ void split_start(SplitStart& st, uint32_t r, uint32_t off, uint32_t len,
-                                            uint32_t pos) {
+// Start inside the sequence of rank r, from_off positions after its first; its
+// pairs take len positions each.
+__device__ __forceinline__ void split_start(SplitStart& st, uint32_t r, uint64_t from_off,
+                                            uint32_t len) {
   st.r = r;
-  st.kvh = (pos - off) / len;
-  st.key = pos - off - st.kvh * len;
+  st.kvh = quotient(from_off, len);
+  st.key = static_cast<uint32_t>(from_off - static_cast<uint64_t>(st.kvh) * len);
 }
 
 // The start of this workgroup, found by itself: thread t holds sequences
@@ -208,14 +234,14 @@ __device__ __forceinline__ bool plan_inline(const DecodeParams& p, SeqEntry* s_e
     cnt += n[j] > 0 ? 1 : 0;
   }
   uint32_t before, rank, all_keys, all_cnt;
-  scan_keys<4, 0>(keys, cnt, before, rank, all_keys, all_cnt);
-  Line L = plan_line(p, all_keys * p.hkv, all_cnt * p.hkv);
+  scan_keys<4, 0, uint32_t>(keys, cnt, before, rank, all_keys, all_cnt);
+  Line<uint32_t> L = plan_line<uint32_t>(p, all_keys * p.hkv, all_cnt * p.hkv);
   before += rank * p.pad;
   if (L.aligned) {
     uint32_t len = 0, none;
 #pragma unroll
     for (int j = 0; j < kInlinePer; ++j) len += L.length(n[j], 0);
-    scan_keys<4, 1>(len, 0, before, none, L.total, none);
+    scan_keys<4, 1, uint32_t>(len, 0, before, none, L.total, none);
     L.total *= p.hkv;
   }
   const uint64_t pos64 = static_cast<uint64_t>(blockIdx.x) * L.share;
@@ -224,15 +250,15 @@ __device__ __forceinline__ bool plan_inline(const DecodeParams& p, SeqEntry* s_e
   for (int j = 0; j < kInlinePer; ++j) {
     const int b = tid * per + j;
     const uint32_t off = before * p.hkv, len = L.length(n[j], p.pad);
-    if (blockIdx.x == 0 && j < per && b < p.batch) p.plan[1 + b] = make_uint4(off, n[j], rank, len);
+    if (blockIdx.x == 0 && j < per && b < p.batch) p.plan[1 + b] = plan_entry(off, n[j], rank, len);
     if (n[j] > 0) {
-      s_ent[rank] = SeqEntry{b, lo[j], n[j], static_cast<int>(len)};
-      if (pos >= off && pos - off < len * p.hkv) split_start(s_start, rank, off, len, pos);
+      s_ent[rank] = SeqEntry{b, lo[j], n[j], len};
+      if (pos >= off && pos - off < len * p.hkv) split_start(s_start, rank, pos - off, len);
       ++rank;
     }
     before += len;
   }
-  if (blockIdx.x == 0 && tid == 0) p.plan[0] = make_uint4(L.share, L.total, 0, 0);
+  if (blockIdx.x == 0 && tid == 0) p.plan[0] = make_uint4(L.share, L.total, 0u, 0u);
   if (pos >= L.total) return false;   // uniform
   __syncthreads();
   st = s_start;
@@ -247,36 +273,39 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(const DecodeP
   const int tid = threadIdx.x;
   const int per = (p.batch + kPlanThreads - 1) / kPlanThreads;
   const int b0 = min(tid * per, p.batch), b1 = min(b0 + per, p.batch);
-  uint32_t keys = 0, cnt = 0;
+  uint64_t keys = 0;
+  uint32_t cnt = 0;
   for (int b = b0; b < b1; ++b) {
     int lo, n;
     key_range(p, b, lo, n);
     keys += n;
     cnt += n > 0 ? 1 : 0;
   }
-  uint32_t before, rank, all_keys, all_cnt;
-  scan_keys<kPlanThreads / 64, 0>(keys, cnt, before, rank, all_keys, all_cnt);
-  Line L = plan_line(p, all_keys * p.hkv, all_cnt * p.hkv);
-  before += rank * p.pad;
+  uint64_t before, all_keys;
+  uint32_t rank, all_cnt;
+  scan_keys<kPlanThreads / 64, 0, uint64_t>(keys, cnt, before, rank, all_keys, all_cnt);
+  Line<uint64_t> L = plan_line<uint64_t>(p, all_keys * p.hkv, all_cnt * p.hkv);
+  before += static_cast<uint64_t>(rank) * p.pad;
   if (L.aligned) {   // few of the sequences hold keys
-    uint32_t len = 0, none;
+    uint64_t len = 0;
+    uint32_t none;
     for (int b = b0; b < b1; ++b) {
       int lo, n;
       key_range(p, b, lo, n);
       len += L.length(n, 0);
     }
-    scan_keys<kPlanThreads / 64, 1>(len, 0, before, none, L.total, none);
+    scan_keys<kPlanThreads / 64, 1, uint64_t>(len, 0, before, none, L.total, none);
     L.total *= p.hkv;
   }
   for (int b = b0; b < b1; ++b) {
     int lo, n;
     key_range(p, b, lo, n);
     const uint32_t len = L.length(n, p.pad);
-    p.plan[1 + b] = make_uint4(before * p.hkv, n, rank, len);
+    p.plan[1 + b] = plan_entry(before * p.hkv, n, rank, len);
     if (n > 0) p.list[rank++] = b;
     before += len;
   }
-  if (tid == 0) p.plan[0] = make_uint4(L.share, L.total, 0, 0);
+  if (tid == 0) p.plan[0] = make_uint4(L.share, static_cast<uint32_t>(L.total), static_cast<uint32_t>(L.total >> 32), 0u);
 }
 
 // The start of this workgroup from the plan kernel's table: a search for the
@@ -284,18 +313,19 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(const DecodeP
 // keys: the sequences after it start later, and one without keys shares its
 // position with the next).  Every thread runs the same search.
 __device__ __forceinline__ bool plan_listed(const DecodeParams& p, SplitStart& st) {
-  const uint32_t share = p.plan[0].x, total = p.plan[0].y;
-  const uint64_t pos64 = static_cast<uint64_t>(blockIdx.x) * share;
-  if (pos64 >= total) return false;
-  const uint32_t pos = static_cast<uint32_t>(pos64);
+  const uint4 line = p.plan[0];
+  const uint32_t share = line.x;
+  const uint64_t total = line.y | static_cast<uint64_t>(line.z) << 32;
+  const uint64_t pos = static_cast<uint64_t>(blockIdx.x) * share;
+  if (pos >= total) return false;
   int lo = 0, hi = p.batch - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (p.plan[1 + mid].x <= pos) lo = mid; else hi = mid - 1;
+    if (seq_place(p.plan[1 + mid]).off <= pos) lo = mid; else hi = mid - 1;
   }
-  const uint4 q = p.plan[1 + lo];
-  split_start(st, q.z, q.x, q.w, pos);
-  st.take = min(total - pos, share);
+  const SeqPlace q = seq_place(p.plan[1 + lo]);
+  split_start(st, q.rank, pos - q.off, q.len);
+  st.take = static_cast<uint32_t>(min(total - pos, static_cast<uint64_t>(share)));
   return true;
 }
 
@@ -331,8 +361,9 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecodeParams p)
   }
   // Workgroup-uniform walk over the pieces, in scalar registers.
   auto uniform = [](uint32_t x) { return static_cast<int>(__builtin_amdgcn_readfirstlane(static_cast<int>(x))); };
-  int r = uniform(st.r), kvh = uniform(st.kvh), key = uniform(st.key);
-  int left = uniform(st.take);   // positions of the line this workgroup still has to take
+  int r = uniform(st.r), kvh = uniform(st.kvh);
+  uint32_t key = uniform(st.key);
+  uint32_t left = uniform(st.take);   // positions of the line this workgroup still has to take
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int kg = lane >> 4, ds = lane & 15;
   const int64_t row_stride = static_cast<int64_t>(p.hkv) * kD;   // elements per cache row
@@ -345,13 +376,14 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecodeParams p)
       key_range(p, e.b, e.lo, e.n);
       e.len = p.plan[1 + e.b].w;
     }
-    const int b = uniform(e.b), n = uniform(e.n), len = uniform(e.len);
-    const int took = min(left, len - key);
+    const int b = uniform(e.b);
+    const uint32_t n = uniform(e.n), len = uniform(e.len);
+    const uint32_t took = min(left, len - key);
     left -= took;
     if (key < n) {   // else this share starts in the pair's padding
     const int64_t slot = static_cast<int64_t>(blockIdx.x) + static_cast<int64_t>(r) * p.hkv + kvh;
     // Piece [k0, k1) of the pair's keys.
-    const int k0 = uniform(e.lo) + key, k1 = k0 + min(took, n - key);
+    const int k0 = uniform(e.lo) + static_cast<int>(key), k1 = k0 + static_cast<int>(min(took, n - key));
     // Q rows of the group: dims 8*ds .. +7 of each head, in fp32, pre-scaled
     // by c so that a dot product is already the exp2-domain score.
     float qv[G][8];
@@ -492,7 +524,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecodeParams p)
     }
     // The rest of the share continues at the start of the next pair (the
     // share ends inside this one otherwise).
-    if (left <= 0) return;
+    if (left == 0u) return;
     key = 0;
     if (++kvh == p.hkv) {
       kvh = 0;
@@ -517,12 +549,12 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const DecodeParams p)
   const int b = static_cast<int>(row / p.hq), hq = static_cast<int>(row - static_cast<int64_t>(b) * p.hq);
   const int kvh = hq / p.group, h = hq - kvh * p.group;
   // The pair's place on the line, the workgroups that share it and its slots.
-  const uint4 seq = p.plan[1 + b];   // line position, keys, rank, positions per pair
+  const SeqPlace seq = seq_place(p.plan[1 + b]);
   const uint32_t share = p.plan[0].x;
-  const uint32_t off = seq.x + kvh * seq.w;
-  const uint32_t wg0 = off / share;
-  const int nch = seq.y > 0 ? static_cast<int>((off + seq.y - 1) / share - wg0) + 1 : 0;   // at most 256
-  const int64_t slot0 = static_cast<int64_t>(wg0) + static_cast<int64_t>(seq.z) * p.hkv + kvh;
+  const uint64_t off = seq.off + static_cast<uint64_t>(kvh) * seq.len;
+  const uint32_t wg0 = quotient(off, share);
+  const int nch = seq.n > 0 ? static_cast<int>(quotient(off + seq.n - 1, share) - wg0) + 1 : 0;   // at most 256
+  const int64_t slot0 = static_cast<int64_t>(wg0) + static_cast<int64_t>(seq.rank) * p.hkv + kvh;
   const int g = tid >> 5, q = tid & 31;
   const float4* base = reinterpret_cast<const float4*>(p.part_o + (slot0 * p.group + h) * kD) + q;
   const int64_t cstride = static_cast<int64_t>(p.group) * (kD / 4);
@@ -641,8 +673,6 @@ static int decode_check(const char* name, const void* q, const void* k_cache,
   if (batch > 65535 || heads_kv > 65535 || cache_len > INT32_MAX ||
       static_cast<int64_t>(batch) * heads_q > INT32_MAX)
     return invalid(n + ": batch, heads_kv or cache_len too large");
-  if (static_cast<int64_t>(batch) * cache_len > INT32_MAX / heads_kv)
-    return invalid(n + ": the K cache holds more rows than any device");
   if (q == nullptr || k_cache == nullptr || v_cache == nullptr || cache_lens == nullptr ||
       full == nullptr || out == nullptr || lse == nullptr)
     return invalid(n + ": null pointer");
@@ -681,6 +711,11 @@ static int decode_launch(const char* name, const void* q, const void* k_cache,
   p.list = reinterpret_cast<int32_t*>(ws + L.off_list);
   p.plan = reinterpret_cast<uint4*>(ws + L.off_plan);
   p.target = kSplitTarget * cus;
+  // A share is at most the line over the resident workgroups, and has to fit 32
+  // bits: with 256 CUs the limit is 128 TiB of K, the size of the address space.
+  const int64_t rows = static_cast<int64_t>(batch) * cache_len * heads_kv;
+  if (rows / p.target >= (int64_t{1} << 30))
+    return invalid(std::string(name) + ": the K cache is larger than the address space");
   // (Padding positions of the line stay below 2^30 beside at most 2^31 keys.)
   p.pad = static_cast<int64_t>(batch) * heads_kv < (int64_t{1} << 30) / kPairPad ? kPairPad : 0;
   p.batch = batch;
@@ -696,8 +731,9 @@ static int decode_launch(const char* name, const void* q, const void* k_cache,
   // Up to kInlineSeqs sequences the split workgroups plan for themselves, at
   // up to kInlinePer sequences per thread; beyond that each of them would
   // read too many lengths and the plan kernel's few us no longer count
-  // beside the thousands of pairs.
-  const bool inline_plan = batch <= kInlineSeqs;
+  // beside the thousands of pairs.  (Caches of 2^31 rows, which only a sparsely
+  // mapped address range can hold, need the plan kernel's 64-bit positions.)
+  const bool inline_plan = batch <= kInlineSeqs && rows <= INT32_MAX;
   if (!inline_plan) hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0, st, p);
   // Grid: one workgroup per share, no more of them than whole caches can fill
   // at kMinShare positions each.
@@ -714,8 +750,8 @@ static int decode_launch(const char* name, const void* q, const void* k_cache,
     case 7: launch_split<7>(inline_plan, grid, st, p); break;
     default: launch_split<8>(inline_plan, grid, st, p); break;
   }
-  const int64_t rows = static_cast<int64_t>(batch) * heads_q;
-  hipLaunchKernelGGL(decode_merge_kernel, dim3(static_cast<uint32_t>(rows)), dim3(256), 0, st, p);
+  const int64_t out_rows = static_cast<int64_t>(batch) * heads_q;
+  hipLaunchKernelGGL(decode_merge_kernel, dim3(static_cast<uint32_t>(out_rows)), dim3(256), 0, st, p);
   return launch_status(name);
 }
 

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import oracle
-from switchattentionkernels_amd import switch_gqa_decode_forward
+from switchattentionkernels_amd import _lib, switch_gqa_decode_forward
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +65,35 @@ def test_decode_line(batch, cache, hq, hkv, w, p, kind):
         assert float(d.max()) <= 2e-2 and float(d.mean()) <= 2e-3
         rel = (lse[live] - lse_r[live]).abs() / lse_r[live].abs().clamp_min(1.0)
         assert float(rel.max()) <= 1e-3
+
+
+@pytest.mark.parametrize("batch,cache", [(3, 1 << 30), (1100, 1 << 22), (2, 2 ** 31 - 1)])
+def test_decode_over_a_sparse_address_range(batch, cache):
+    """Caches of more than 2^31 rows of address range, of which only the first
+    sequence's are there and only they have keys, as a caller that maps its
+    cache by need can have through the C ABI: the plan's positions are 64-bit
+    for these."""
+    hq, hkv, w, n = 8, 2, 100, 300
+    gen = torch.Generator().manual_seed(batch)
+    q = torch.randn(batch, hq, 128, generator=gen).bfloat16().to(DEV)
+    k, v = (torch.randn(1, n, hkv, 128, generator=gen).bfloat16().to(DEV) for _ in range(2))
+    full = torch.ones(batch, dtype=torch.bool, device=DEV)
+    lens = torch.zeros(batch, dtype=torch.int32, device=DEV)
+    lens[0] = n
+    assert batch * cache * hkv > 2 ** 31
+    L = _lib.lib()
+    need = L.swattn_decode_workspace_bytes(batch, cache, hq, hkv)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    o = torch.empty_like(q)
+    lse = torch.empty(batch, hq, device=DEV)
+    print(f"[decode line] B{batch} L{cache} sparse", flush=True)
+    st = L.swattn_decode_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), lens.data_ptr(),
+                             full.data_ptr(), o.data_ptr(), lse.data_ptr(), batch, cache, hq, hkv,
+                             128, w, 128 ** -0.5 * 1.4426950408889634, ws.data_ptr(), need,
+                             _lib.stream_handle(DEV))
+    assert st == 0, L.swattn_last_error()
+    o_r, lse_r = oracle.decode_attention(q[:1].cpu(), k.cpu(), v.cpu(), [n], [True], window_size=w)
+    d = (o[0].float().cpu() - o_r.float().view(hq, 128)).abs()
+    assert float(d.max()) <= 2e-2 and float(d.mean()) <= 2e-3
+    assert torch.allclose(lse[0].cpu(), lse_r.view(hq), rtol=1e-3)
+    assert bool(torch.isnan(o[1:]).all()) and bool((lse[1:] == -torch.inf).all())
