@@ -645,7 +645,7 @@ static DecodeLayout decode_layout(int64_t batch, int64_t heads_q, int64_t heads_
   auto al = [](int64_t x) { return (x + 255) & ~static_cast<int64_t>(255); };
   int64_t o = al(L.slots * group * kD * 4);               // part_o
   L.off_ml = o;    o = al(o + L.slots * group * 2 * 4);
-  L.off_list = o;  o = al(o + L.slots * 8);
+  L.off_list = o;  o = al(o + batch * 4);
   L.off_plan = o;  o = al(o + (1 + batch) * 16);
   L.bytes = o;
   return L;
@@ -787,7 +787,7 @@ int swattn_decode_fwd(const void* q, const void* k_cache, const void* v_cache,
 // host-side stand-in, so its device address is looked up once per device
 // (hipGetSymbolAddress, with that device current) and only that address is
 // ever handed to kernels.  The decode kernels write every scratch byte they
-// read within the same call (plan, work items, split partials), so nothing
+// read within the same call (plan, list of sequences, partials), so nothing
 // needs clearing between calls; two calls that overlap on one GPU share the
 // array and race.
 // ---------------------------------------------------------------------------

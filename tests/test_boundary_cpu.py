@@ -110,6 +110,22 @@ def test_version_and_workspace():
     assert lib.swattn_prefill_bwd_workspace_bytes(1, 1000, 32, 8, 128, 0, 300, 700) == 0
 
 
+def test_decode_workspace_holds_partials_list_and_plan():
+    """Per slot (four per CU, one per (sequence, KV head)) G fp32 output rows and
+    G (maximum, sum) pairs; the list of sequences, one int32 each; the plan, 16
+    bytes per sequence and one record more.  Each part is 256-byte aligned."""
+    lib = _lib.lib()
+
+    def al(x):
+        return -(-x // 256) * 256
+
+    cus = 256   # also what the library assumes where it finds no device
+    for batch, hq, hkv in ((1, 8, 8), (64, 32, 8), (1025, 8, 1), (5000, 16, 2)):
+        slots, g = 4 * cus + batch * hkv, hq // hkv
+        want = al(slots * g * 512) + al(slots * g * 8) + al(4 * batch) + al(16 * (1 + batch))
+        assert lib.swattn_decode_workspace_bytes(batch, 100, hq, hkv) == want
+
+
 def test_host_side_argument_errors():
     lib = _lib.lib()
     # head_dim != 128
