@@ -21,6 +21,7 @@ namespace {
 
 using at::Tensor;
 using std::optional;
+namespace py = pybind11;
 
 void check(int status, const char* what) {
   TORCH_CHECK(status == SWATTN_OK, what, " failed with status ", status, ": ", swattn_last_error());
@@ -74,8 +75,14 @@ std::tuple<Tensor, Tensor> compact(const Tensor& x, int64_t dtype, double thresh
 }
 
 // Whether q, k, v meet every precondition of the prefill (the Python layer
-// finds out which one fails and raises for it).
-bool qkv_ok(const Tensor& q, const Tensor& k, const Tensor& v) {
+// finds out which one fails and raises for it, also for arguments that are no
+// tensors).
+bool qkv_ok(const py::object& qo, const py::object& ko, const py::object& vo) {
+  if (!THPVariable_Check(qo.ptr()) || !THPVariable_Check(ko.ptr()) || !THPVariable_Check(vo.ptr()))
+    return false;
+  const Tensor& q = THPVariable_Unpack(qo.ptr());
+  const Tensor& k = THPVariable_Unpack(ko.ptr());
+  const Tensor& v = THPVariable_Unpack(vo.ptr());
   return q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 &&
          v.scalar_type() == at::kBFloat16 && q.is_cuda() && k.is_cuda() && v.is_cuda() &&
          q.layout() == at::kStrided && k.layout() == at::kStrided && v.layout() == at::kStrided &&

@@ -1,0 +1,28 @@
+"""The native extension's edges that need no GPU: how its errors reach Python,
+what its checks leave to the Python layer, and what a missing or unusable
+build says."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from switchattentionkernels_amd import _lib, switch_gqa_prefill_forward
+
+
+def test_errors_carry_the_message_alone():
+    """A refused call raises RuntimeError with the status and the library's
+    message, as the ctypes calls do, and no C++ stack trace."""
+    x = torch.zeros(1, 1, 2, 128, dtype=torch.bfloat16)
+    idx = torch.zeros(1, dtype=torch.int32)
+    with pytest.raises(RuntimeError) as e:   # refused on the host: the window
+        _lib.native().prefill_forward(x, x, x, idx, idx[:0], None, None, None, 0, 0.1, 0)
+    assert str(e.value) == ("swattn_prefill_fwd failed with status -1: "
+                            "swattn_prefill_fwd: window must be positive")
+
+
+def test_arguments_that_are_no_tensors_reach_the_python_checks():
+    a = np.zeros((1, 4, 2, 128), dtype=np.float32)
+    with pytest.raises(TypeError, match="requires BF16"):
+        switch_gqa_prefill_forward(a, a, a, None, None)
