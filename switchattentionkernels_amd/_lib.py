@@ -65,8 +65,13 @@ def native():
             spec = importlib.util.spec_from_file_location(
                 "_native", NATIVE_PATH,
                 loader=importlib.machinery.ExtensionFileLoader("_native", NATIVE_PATH))
-            mod = importlib.util.module_from_spec(spec)
-            spec.loader.exec_module(mod)
+            try:
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+            except ImportError as e:
+                raise LibraryNotBuilt(
+                    f"{NATIVE_PATH} cannot be loaded by this Python and torch ({e}): build it "
+                    "again with `python -m switchattentionkernels_amd.build`") from e
             _native = mod
     return _native
 

@@ -26,3 +26,15 @@ def test_arguments_that_are_no_tensors_reach_the_python_checks():
     a = np.zeros((1, 4, 2, 128), dtype=np.float32)
     with pytest.raises(TypeError, match="requires BF16"):
         switch_gqa_prefill_forward(a, a, a, None, None)
+
+
+@pytest.mark.parametrize("content", [None, b"not a shared library"])
+def test_missing_or_unusable_extension_says_so(monkeypatch, tmp_path, content):
+    """No extension, or one that this Python or torch cannot load."""
+    path = tmp_path / "_native.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "NATIVE_PATH", str(path))
+    with pytest.raises(_lib.LibraryNotBuilt, match="switchattentionkernels_amd.build"):
+        _lib.native()
