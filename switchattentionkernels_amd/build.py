@@ -80,10 +80,11 @@ def generate_sources() -> None:
 
 
 def build(verbose: bool = False, out: str = LIB, extra_flags=(), sources=None) -> str:
-    """Compile ``libswattn.so`` (or ``out``, with ``extra_flags`` appended to
-    the compile flags; ``sources`` relative to ``csrc/``, default the
-    attention library's); returns its path.  Always regenerates the
-    generated includes and recompiles."""
+    """Compile ``libswattn.so`` and the extension that the package calls it
+    with, ``_native.so``; returns the library's path.  With ``out``: only that
+    library, with ``extra_flags`` appended to the compile flags and
+    ``sources`` relative to ``csrc/`` (default the attention library's).
+    Always regenerates the generated includes and recompiles."""
     generate_sources()
     cmd = [_hipcc()] + compile_flags() + list(extra_flags)
     tl = _torch_lib_dir()
@@ -102,6 +103,8 @@ def build(verbose: bool = False, out: str = LIB, extra_flags=(), sources=None) -
     if verbose and err:
         print(err, file=sys.stderr)
     os.replace(tmp, out)
+    if out == LIB:
+        build_native(verbose=verbose)
     return out
 
 
@@ -165,6 +168,5 @@ def build_c_caller(verbose: bool = False) -> str:
 
 if __name__ == "__main__":
     print(build(verbose=True))
-    print(build_native(verbose=True))
     print(build_probe(verbose=True))
     print(build_c_caller(verbose=True))

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from switchattentionkernels_amd import _lib, switch_gqa_prefill_forward
+from switchattentionkernels_amd import _lib, build as B, switch_gqa_prefill_forward
 
 
 def test_errors_carry_the_message_alone():
@@ -38,3 +38,21 @@ def test_missing_or_unusable_extension_says_so(monkeypatch, tmp_path, content):
     monkeypatch.setattr(_lib, "NATIVE_PATH", str(path))
     with pytest.raises(_lib.LibraryNotBuilt, match="switchattentionkernels_amd.build"):
         _lib.native()
+
+
+def test_build_makes_a_usable_package(monkeypatch):
+    """``build()`` alone compiles the library and the extension that loads it."""
+    made = []
+
+    class Done:
+        returncode, stderr = 0, ""
+
+    monkeypatch.setattr(B, "generate_sources", lambda: None)
+    monkeypatch.setattr(B.subprocess, "run", lambda cmd, **kw: made.append(cmd) or Done())
+    monkeypatch.setattr(B.os, "replace", lambda a, b: None)
+    assert B.build() == B.LIB
+    outs = [cmd[cmd.index("-o") + 1] for cmd in made]
+    assert outs == [B.LIB + ".tmp", B.NATIVE_LIB + ".tmp"]
+    made.clear()
+    B.build(out="/elsewhere/lib.so")   # a library of its own, such as an instrumented one
+    assert len(made) == 1
