@@ -15,7 +15,8 @@ import importlib.util
 import os
 import threading
 
-import torch  # noqa: F401  -- loads PyTorch's HIP runtime before the library
+import torch  # loads PyTorch's HIP runtime before the library
+from torch.overrides import has_torch_function_unary
 
 from ._abi import INTERNAL_SIGNATURES, PROBE_SIGNATURES, SIGNATURES, bind  # noqa: F401  -- API
 
@@ -97,6 +98,12 @@ def check(status: int, what: str) -> None:
 def ptr(t) -> int | None:
     """Device address of a tensor (None for None)."""
     return None if t is None else t.data_ptr()
+
+
+def like(t):
+    """``torch.empty_like(t)`` where a tensor subclass or a function mode may have
+    a say in it, else None: the native layer allocates the output itself."""
+    return torch.empty_like(t) if has_torch_function_unary(t) else None
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

@@ -99,7 +99,8 @@ def switch_gqa_prefill_backward(
     with _lib.on_device(q.device):
         return _lib.native().prefill_backward(q, k, v, output, lse, grad_output, full, local, fs,
                                               ls, ends, int(window_size), scale * LOG2E,
-                                              _lib.stream_handle(q.device))
+                                              _lib.stream_handle(q.device), _lib.like(q),
+                                              _lib.like(k), _lib.like(v))
 
 
 class SwitchGQAPrefillFunction(torch.autograd.Function):

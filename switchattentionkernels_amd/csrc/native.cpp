@@ -33,6 +33,12 @@ Tensor bytes(const Tensor& like, size_t n) {
   return at::empty({static_cast<int64_t>(n)}, like.options().dtype(at::kByte));
 }
 
+// An output like t: the one that the Python layer made, where a tensor subclass
+// has a say in that, or a new one.
+Tensor like(const Tensor& t, const optional<Tensor>& made) {
+  return made.has_value() ? *made : at::empty(t.sizes(), t.options());
+}
+
 const int32_t* i32(const Tensor& t) { return static_cast<const int32_t*>(t.const_data_ptr()); }
 const int32_t* i32(const optional<Tensor>& t) { return t.has_value() ? i32(*t) : nullptr; }
 
@@ -97,11 +103,12 @@ std::tuple<Tensor, Tensor> prefill_forward(const Tensor& q, const Tensor& k, con
                                            const optional<Tensor>& full_starts,
                                            const optional<Tensor>& local_starts,
                                            const optional<Tensor>& causal_ends, int64_t window,
-                                           double scale_log2, int64_t stream) {
+                                           double scale_log2, int64_t stream,
+                                           const optional<Tensor>& out_made) {
   const int32_t batch = static_cast<int32_t>(q.size(0)), hq = static_cast<int32_t>(q.size(2));
   const int32_t hkv = static_cast<int32_t>(k.size(2)), dim = static_cast<int32_t>(q.size(3));
   const int64_t sq = q.size(1), skv = k.size(1), nf = full.numel(), nl = local.numel();
-  const Tensor out = at::empty(q.sizes(), q.options());
+  const Tensor out = like(q, out_made);
   const Tensor lse = at::empty({q.size(0), sq, q.size(2)}, q.options().dtype(at::kFloat));
   const int32_t w = static_cast<int32_t>(window);
   // The larger workspace that lets the kernel split long full items by key
@@ -126,14 +133,15 @@ std::tuple<Tensor, Tensor, Tensor> prefill_backward(
     const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
     const Tensor& grad, const Tensor& full, const Tensor& local,
     const optional<Tensor>& full_starts, const optional<Tensor>& local_starts,
-    const optional<Tensor>& causal_ends, int64_t window, double scale_log2, int64_t stream) {
+    const optional<Tensor>& causal_ends, int64_t window, double scale_log2, int64_t stream,
+    const optional<Tensor>& dq_made, const optional<Tensor>& dk_made,
+    const optional<Tensor>& dv_made) {
   const int32_t batch = static_cast<int32_t>(q.size(0)), hq = static_cast<int32_t>(q.size(2));
   const int32_t hkv = static_cast<int32_t>(k.size(2)), dim = static_cast<int32_t>(q.size(3));
   const int64_t sq = q.size(1), skv = k.size(1), nf = full.numel(), nl = local.numel();
   // The lists cover every query position once (checked by the caller), and the
   // kernels write every listed row (0 for a row with no key): no fill.
-  const Tensor dq = at::empty(q.sizes(), q.options()), dk = at::empty(k.sizes(), k.options()),
-               dv = at::empty(v.sizes(), v.options());
+  const Tensor dq = like(q, dq_made), dk = like(k, dk_made), dv = like(v, dv_made);
   const int32_t w = static_cast<int32_t>(window);
   const size_t ws_bytes = swattn_prefill_bwd_workspace_bytes(batch, skv, hq, hkv, dim, w, nf, nl);
   const Tensor ws = bytes(q, ws_bytes > 0 ? ws_bytes : 1);
@@ -154,10 +162,11 @@ std::tuple<Tensor, Tensor, Tensor> prefill_backward(
 
 std::tuple<Tensor, Tensor> decode_forward(const Tensor& q, const Tensor& k, const Tensor& v,
                                           const Tensor& lens, const Tensor& full, int64_t window,
-                                          double scale_log2, int64_t stream) {
+                                          double scale_log2, int64_t stream,
+                                          const optional<Tensor>& out_made) {
   const int32_t batch = static_cast<int32_t>(q.size(0)), hq = static_cast<int32_t>(q.size(2));
   const int32_t hkv = static_cast<int32_t>(k.size(2)), dim = static_cast<int32_t>(q.size(3));
-  const Tensor out = at::empty(q.sizes(), q.options());
+  const Tensor out = like(q, out_made);
   const Tensor lse = at::empty({q.size(0), 1, q.size(2)}, q.options().dtype(at::kFloat));
   const size_t ws_bytes = swattn_decode_workspace_bytes(batch, k.size(1), hq, hkv);
   const Tensor ws = bytes(q, ws_bytes);

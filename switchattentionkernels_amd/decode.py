@@ -68,7 +68,7 @@ def switch_gqa_decode_forward(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     full = full_mask.contiguous()
     with _lib.on_device(dev):
         out, lse = _lib.native().decode_forward(q, k_cache, v_cache, lens, full, int(window_size),
-                                                scale, _lib.stream_handle(dev))
+                                                scale, _lib.stream_handle(dev), _lib.like(q))
     if squeeze:
         return out[:, 0], lse[:, 0]
     return out, lse

@@ -304,7 +304,7 @@ def switch_gqa_prefill_forward(
         metadata.full_starts, metadata.local_starts, metadata.causal_ends)
     with _lib.on_device(q.device):
         return _lib.native().prefill_forward(q, k, v, full, local, fs, ls, ends, int(window_size),
-                                             scale, _lib.stream_handle(q.device))
+                                             scale, _lib.stream_handle(q.device), _lib.like(q))
 
 
 def switch_gqa_prefill_varlen_forward(

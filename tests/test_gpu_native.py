@@ -1,0 +1,69 @@
+"""What the native host path keeps of the calls' behaviour in Python: the type
+of a tensor subclass, torch's out-of-memory error, torch's synchronization
+debug mode, and metadata fields that are tensors of their own."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from switchattentionkernels_amd import (build_switch_attention_metadata,
+                                        build_switch_query_indices,
+                                        build_switch_query_indices_from_logits,
+                                        switch_gqa_decode_forward, switch_gqa_prefill_backward,
+                                        switch_gqa_prefill_forward)
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+
+
+class Tagged(torch.Tensor):
+    pass
+
+
+def _qkv(s=200, hq=8, hkv=2):
+    return [torch.randn(1, s, h, 128, device=DEV).bfloat16() for h in (hq, hkv, hkv)]
+
+
+def _lists(s=200):
+    return build_switch_query_indices(torch.arange(s, device=DEV) % 3 == 0)
+
+
+def test_subclasses_come_back():
+    """Outputs are made like the tensors they belong to, as torch.empty_like makes them."""
+    q, k, v = _qkv()
+    full, local = _lists()
+    tq, tk = q.as_subclass(Tagged), k.as_subclass(Tagged)
+    o, lse = switch_gqa_prefill_forward(q, k, v, full, local, window_size=50)
+    to, tlse = switch_gqa_prefill_forward(tq, tk, v, full, local, window_size=50)
+    assert type(o) is torch.Tensor and type(to) is Tagged
+    assert type(lse) is torch.Tensor and type(tlse) is torch.Tensor
+    assert torch.equal(o, to.as_subclass(torch.Tensor)) and torch.equal(lse, tlse)
+    want = switch_gqa_prefill_backward(q, k, v, o, lse, q, full, local, window_size=50)
+    got = switch_gqa_prefill_backward(tq, tk, v, o, lse, q, full, local, window_size=50)
+    assert [type(t) for t in got] == [Tagged, Tagged, torch.Tensor]
+    for a, b in zip(want, got):
+        assert torch.equal(a, b.as_subclass(torch.Tensor))
+    lens = torch.tensor([200], dtype=torch.int32, device=DEV)
+    route = torch.ones(1, dtype=torch.bool, device=DEV)
+    for qd in (q[:, -1:].contiguous(), q[:, -1].contiguous()):
+        o, _ = switch_gqa_decode_forward(qd, k, v, lens, route)
+        to, _ = switch_gqa_decode_forward(qd.as_subclass(Tagged), k, v, lens, route)
+        assert type(to) is Tagged and torch.equal(o, to.as_subclass(torch.Tensor))
+
+
+def test_out_of_memory_is_torchs_error():
+    q, k, v = _qkv(s=65536, hq=8, hkv=8)   # 128 MiB each
+    full, local = _lists(65536)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2 ** 20) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            switch_gqa_prefill_forward(q, k, v, full, local)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    o, _ = switch_gqa_prefill_forward(q, k, v, full, local)
+    assert bool(torch.isfinite(o).all())

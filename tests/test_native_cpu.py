@@ -17,7 +17,7 @@ def test_errors_carry_the_message_alone():
     x = torch.zeros(1, 1, 2, 128, dtype=torch.bfloat16)
     idx = torch.zeros(1, dtype=torch.int32)
     with pytest.raises(RuntimeError) as e:   # refused on the host: the window
-        _lib.native().prefill_forward(x, x, x, idx, idx[:0], None, None, None, 0, 0.1, 0)
+        _lib.native().prefill_forward(x, x, x, idx, idx[:0], None, None, None, 0, 0.1, 0, None)
     assert str(e.value) == ("swattn_prefill_fwd failed with status -1: "
                             "swattn_prefill_fwd: window must be positive")
 
