@@ -113,6 +113,16 @@ def _raise_for(flags: int, which: str) -> None:
             raise ValueError(MSG_ORDER)
 
 
+_sync_debug_mode = getattr(torch._C, "_cuda_get_sync_debug_mode", torch.cuda.get_sync_debug_mode)
+
+
+def _note_sync(device) -> None:
+    """The compaction waits for its counts without torch's knowledge: in torch's
+    synchronization debug mode a read of torch's own warns or raises for it."""
+    if _sync_debug_mode():
+        torch.empty(1, dtype=torch.int32, device=device).item()
+
+
 class _Compaction:
     """Identity of one ``build_switch_query_indices`` result (``n`` positions)."""
 
@@ -194,8 +204,8 @@ def build_switch_query_indices(full_mask: torch.Tensor) -> Tuple[torch.Tensor, t
     ``[0, S)``; a ``[B, S]`` mask (an extension: V:314-315 rejects B > 1) gives
     flattened positions ``b * S + i``.  Both lists are ascending int32 device
     tensors, bit-identical to ``arange(n)[mask]`` and ``arange(n)[~mask]``.
-    One device-to-host read fetches the split point, as torch's boolean
-    indexing does in the reference.
+    The call waits for the split point, as torch's boolean indexing does in the
+    reference.
     """
     if full_mask.ndim == 2:
         full_mask = full_mask.reshape(-1)
@@ -208,6 +218,7 @@ def build_switch_query_indices(full_mask: torch.Tensor) -> Tuple[torch.Tensor, t
         raise ValueError("full_mask must hold fewer than 2^31 positions")
     dev = full_mask.device
     mask = full_mask.contiguous()
+    _note_sync(dev)
     with _lib.on_device(dev):
         full, local = _lib.native().compact(mask, -1, 0.0, _lib.stream_handle(dev))
     _tag_compacted(full, local, n)
@@ -245,6 +256,7 @@ def build_switch_query_indices_from_logits(
     thr = float(threshold)
     if thr != 0.0 and logits.dtype != torch.float32:   # fp32 is rounded by the call
         thr = float(torch.tensor(thr, dtype=logits.dtype).item())
+    _note_sync(dev)
     with _lib.on_device(dev):
         full, local = _lib.native().compact(logits, _LOGIT_DTYPES[logits.dtype], thr,
                                             _lib.stream_handle(dev))

@@ -67,3 +67,21 @@ def test_out_of_memory_is_torchs_error():
         torch.cuda.set_per_process_memory_fraction(1.0)
     o, _ = switch_gqa_prefill_forward(q, k, v, full, local)
     assert bool(torch.isfinite(o).all())
+
+
+@pytest.mark.parametrize("make", [
+    lambda m: build_switch_query_indices(m),
+    lambda m: build_switch_query_indices_from_logits(m.float(), 0.5)])
+def test_sync_debug_mode_sees_the_wait(make):
+    mask = torch.arange(5000, device=DEV) % 3 == 0
+    make(mask)
+    try:
+        torch.cuda.set_sync_debug_mode("error")
+        with pytest.raises(RuntimeError, match="synchroniz"):
+            make(mask)
+        torch.cuda.set_sync_debug_mode("warn")
+        with pytest.warns(UserWarning, match="synchroniz"):
+            full, local = make(mask)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    assert full.numel() == 1667 and local.numel() == 3333
