@@ -13,6 +13,7 @@
 
 #include <string>
 #include <tuple>
+#include <vector>
 
 #include "swattn.h"
 #include "swattn_internal.h"
@@ -129,6 +130,25 @@ std::tuple<Tensor, Tensor> prefill_forward(const Tensor& q, const Tensor& k, con
   return {out, lse};
 }
 
+// The seven fields of a SwitchAttentionMetadata, in its order; the sequences'
+// offsets, checked and at most SWATTN_METADATA_HOST_MAX_SEQS of them, travel as
+// kernel arguments.
+std::vector<Tensor> metadata(const std::vector<int32_t>& cu_q, const std::vector<int32_t>& cu_kv,
+                             int64_t q_len, int64_t kv_len, int64_t window, at::Device device,
+                             int64_t stream) {
+  const auto opts = at::TensorOptions().dtype(at::kInt).device(device);
+  std::vector<Tensor> f;
+  f.reserve(7);
+  for (const int64_t n : {q_len, kv_len, q_len, kv_len, q_len, q_len, q_len})
+    f.push_back(at::empty({n}, opts));
+  auto out = [&](int i) { return f[i].data_ptr<int32_t>(); };
+  check(swattn_build_metadata_host(cu_q.data(), cu_kv.data(), static_cast<int32_t>(cu_q.size()) - 1,
+                                   q_len, kv_len, static_cast<int32_t>(window), out(0), out(1),
+                                   out(2), out(3), out(4), out(5), out(6), as_stream(stream)),
+        "swattn_build_metadata");
+  return f;
+}
+
 std::tuple<Tensor, Tensor, Tensor> prefill_backward(
     const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
     const Tensor& grad, const Tensor& full, const Tensor& local,
@@ -189,6 +209,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("compact", &compact);
   m.def("qkv_ok", &qkv_ok);
   m.def("prefill_forward", &prefill_forward);
+  m.def("metadata", &metadata);
   m.def("prefill_backward", &prefill_backward);
   m.def("decode_forward", &decode_forward);
 }

@@ -16,7 +16,6 @@ packed sequence, so attention never crosses a sequence boundary.
 
 from __future__ import annotations
 
-import ctypes
 from dataclasses import dataclass
 
 import torch
@@ -79,27 +78,20 @@ def build_switch_attention_metadata(q_len: int, kv_len: int, *, device, window_s
     ck = _as_cu(ck_src, kv_len, "cu_seqlens_kv")
     if len(ck) != len(cq):
         raise ValueError("cu_seqlens and cu_seqlens_kv must describe the same number of sequences")
-    if q_len == kv_len:
-        # One allocation; the fields are its rows.
-        md = SwitchAttentionMetadata(*torch.empty((7, q_len), dtype=torch.int32, device=dev)
-                                     .unbind(0))
-    else:
-        md = SwitchAttentionMetadata(*(torch.empty(n, dtype=torch.int32, device=dev) for n in
-                                       (q_len, kv_len, q_len, kv_len, q_len, q_len, q_len)))
     L, nseq = _lib.lib(), len(cq) - 1
-    outs = [t.data_ptr() for t in (md.q_positions, md.kv_positions, md.q_segment_ids,
-                                   md.kv_segment_ids, md.full_starts, md.local_starts,
-                                   md.causal_ends)]
     with _lib.on_device(dev):
         stream = _lib.stream_handle(dev)
-        if nseq <= HOST_MAX_SEQS:   # the offsets travel as kernel arguments
-            arr = ctypes.c_int32 * (nseq + 1)
-            st = L.swattn_build_metadata_host(arr(*cq), arr(*ck), nseq, q_len, kv_len,
-                                              window_size, *outs, stream)
-        else:
-            cq_t = torch.tensor(cq, dtype=torch.int32, device=dev)
-            ck_t = torch.tensor(ck, dtype=torch.int32, device=dev)
-            st = L.swattn_build_metadata(cq_t.data_ptr(), ck_t.data_ptr(), nseq, q_len, kv_len,
-                                         window_size, *outs, stream)
+        if nseq <= HOST_MAX_SEQS and max(q_len, kv_len) < 2 ** 31:
+            return SwitchAttentionMetadata(*_lib.native().metadata(cq, ck, q_len, kv_len,
+                                                                   window_size, dev, stream))
+        md = SwitchAttentionMetadata(*(torch.empty(n, dtype=torch.int32, device=dev) for n in
+                                       (q_len, kv_len, q_len, kv_len, q_len, q_len, q_len)))
+        cq_t = torch.tensor(cq, dtype=torch.int32, device=dev)
+        ck_t = torch.tensor(ck, dtype=torch.int32, device=dev)
+        st = L.swattn_build_metadata(cq_t.data_ptr(), ck_t.data_ptr(), nseq, q_len, kv_len,
+                                     window_size, *(t.data_ptr() for t in (
+                                         md.q_positions, md.kv_positions, md.q_segment_ids,
+                                         md.kv_segment_ids, md.full_starts, md.local_starts,
+                                         md.causal_ends)), stream)
     _lib.check(st, "swattn_build_metadata")
     return md

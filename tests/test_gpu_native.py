@@ -85,3 +85,23 @@ def test_sync_debug_mode_sees_the_wait(make):
     finally:
         torch.cuda.set_sync_debug_mode("default")
     assert full.numel() == 1667 and local.numel() == 3333
+
+
+@pytest.mark.parametrize("nseq", [1, 7, 256, 257])
+@pytest.mark.parametrize("extra", [0, 3])
+def test_metadata_fields_are_tensors_of_their_own(nseq, extra):
+    """Whole storages, aligned as torch allocates, with version counters of their own."""
+    n = 5 * nseq + 2
+    cu = [5 * i for i in range(nseq)] + [n]
+    ck = cu[:-1] + [n + extra]
+    md = build_switch_attention_metadata(n, n + extra, device=DEV, window_size=3, cu_seqlens=cu,
+                                         cu_seqlens_kv=ck)
+    fields = (md.q_positions, md.kv_positions, md.q_segment_ids, md.kv_segment_ids,
+              md.full_starts, md.local_starts, md.causal_ends)
+    assert len({t.untyped_storage().data_ptr() for t in fields}) == 7
+    for t in fields:
+        assert t.data_ptr() % 256 == 0 and t.storage_offset() == 0
+        assert t.untyped_storage().nbytes() == 4 * t.numel()
+    before = [t._version for t in fields]
+    md.causal_ends.add_(0)
+    assert [t._version for t in fields] == before[:-1] + [before[-1] + 1]
