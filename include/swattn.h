@@ -232,8 +232,10 @@ int swattn_merge_partials(const void* const* o_parts, const float* const* lse_pa
  *   which depends on the current device's CU count (ask on that device).
  * The routed keys of all (sequence, KV head) pairs are shared out evenly over
  * the chip's workgroups, planned on the device from the lengths and routes;
- * fp32 partials are merged by a second kernel.  (More than 1024 sequences: a
- * one-workgroup kernel plans first.)
+ * fp32 partials are merged by a second kernel.  (More than 1024 sequences, or a
+ * cache of 2^31 rows of address range and more: a one-workgroup kernel plans
+ * first.  Refused is a cache larger than the address space, 2^30 rows per
+ * resident workgroup.)
  */
 size_t swattn_decode_workspace_bytes(int32_t batch, int64_t cache_len, int32_t heads_q,
                                      int32_t heads_kv);

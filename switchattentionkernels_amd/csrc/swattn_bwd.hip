@@ -47,7 +47,7 @@
 //   dQ's fill the CUs that dK/dV's leave, and small grids run both at once.
 //   Grids of fewer than 512 (key tile, KV head) pairs may cut a pair over its
 //   row blocks (up to 16 workgroups) where it would outlast the grid's time per
-//   CU.  Pairs run longest first (the first key tiles of each sequence are seen
+//   CU (dkv_chunk).  Pairs run longest first (the first key tiles of each sequence are seen
 //   by the most rows).  When the longest dQ row tile (the latest full rows see
 //   every earlier key) would set dQ's length, row tiles longer than the
 //   estimated key tiles per workgroup slot are cut into equal pieces of their

@@ -718,8 +718,9 @@ def test_decode_plan_with_long_mixed_caches():
 
 
 def test_decode_plan_beyond_lds_sequence_table():
-    """More sequences (5000) than the plan kernel keeps in LDS (4096): the
-    work-item search then runs over the plan in global memory."""
+    """More sequences (5000) than the workgroups plan by themselves (1024):
+    the plan kernel leaves their places on the line in global memory, where
+    every workgroup searches for its start."""
     gen = torch.Generator().manual_seed(78)
     b, cache_len, hq, hkv, w = 5000, 96, 8, 2, 40
     q = torch.randn(b, hq, 128, generator=gen).to(torch.bfloat16)

@@ -1,12 +1,13 @@
-"""The backward's 64-key-per-wave dK/dV kernel (bwd_dkdv_wide_kernel)
-against the oracle and against the eight-wave dK/dV kernel.
+"""The backward's 64-key-per-wave dK/dV product (dkdv_wide, a branch of
+bwd_wide_kernel) against the oracle and against the eight-wave kernel
+(bwd_dkdv_kernel).
 
-The 64-key kernel is the default; under 512 (key tile, KV head) pairs it
-shares each pair's row blocks out over several workgroups whose fp32
-partials the reduce kernel adds, as the eight-wave kernel does.
-SWATTN_DKDV_KERNEL=wide names it explicitly on the small shapes below (all
-split), =narrow forces the eight-wave kernel.  Both take the same split and
-the same dQ kernel, so dq agrees bit for bit.  Their dk and dv differ in
+The 64-key product is the default; under 512 (key tile, KV head) pairs both
+forms cut the long pairs' row blocks over several workgroups whose fp32
+partials bwd_reduce_kernel adds (test_gpu_bwd_cut.py looks at which).
+SWATTN_DKDV_KERNEL=wide names it explicitly on the small shapes below,
+=narrow forces the eight-wave kernel.  Both take the same cuts and
+the same dQ product, so dq agrees bit for bit.  Their dk and dv differ in
 rounding only:
 the 64-key kernel takes a pair's full-branch row blocks from the last down
 (the eight-wave kernel from the first up), so the fp32 sums run in another
@@ -96,15 +97,16 @@ def test_wide_dkdv_varlen_metadata(monkeypatch):
 
 
 @pytest.mark.parametrize("b,s,hq,hkv,w,p", [
-    (1, 8192, 16, 16, 512, 0.3),     # 32 key tiles x 16 KV heads = 512 pairs: no split
+    (1, 8192, 16, 16, 512, 0.3),     # 32 key tiles x 16 KV heads = 512 pairs: never cut
     (2, 4096, 32, 16, 300, 0.5),     # two sequences, 512 pairs
-    (2, 4096, 32, 8, 1024, 0.25),    # 256 pairs: split in two
-    (1, 16384, 4, 1, 1024, 0.25),    # one KV head, 64 pairs: split in eight
-    (1, 1024, 8, 2, 256, 0.25),      # 8 pairs: the largest split
+    (2, 4096, 32, 8, 1024, 0.25),    # 256 pairs, all shorter than the grid's time per CU: whole
+    (2, 2048, 8, 4, 256, 0.9),       # two sequences in turn, 64 pairs, long ones in a few shares
+    (1, 16384, 4, 1, 1024, 0.25),    # one KV head, 64 pairs, up to eight shares
+    (1, 1024, 8, 2, 256, 0.25),      # 8 pairs, up to sixteen shares
 ])
 def test_wide_dkdv_matches_eight_wave(monkeypatch, b, s, hq, hkv, w, p):
-    """The default (64-key) kernel's dk and dv match the eight-wave
-    kernel's within the bar above (dq bit for bit), split or not, and reruns
+    """The default (64-key) product's dk and dv match the eight-wave
+    kernel's within the bar above (dq bit for bit), cut or not, and reruns
     are bit-identical."""
     q, k, v, do = _qkv(b * 7 + s, b, s, hq, hkv)
     m = _mask(s + 9, (b, s), p)

@@ -1,5 +1,6 @@
-"""The backward's 256-row dQ kernel (bwd_dq_wide_kernel, the default) against
-the 32-row-wave dQ kernel (SWATTN_DQ_KERNEL=narrow) and the oracle.
+"""The backward's 256-row dQ product (dq_wide, a branch of bwd_wide_kernel and
+the default) against the 32-row-wave kernel (bwd_dq_kernel,
+SWATTN_DQ_KERNEL=narrow) and the oracle.
 
 Both kernels compute P = 2^(c s - LSE) with the same fp32 operations and
 accumulate S and dQ in the same k-step order.  The 256-row kernel starts
