@@ -60,11 +60,18 @@ def test_out_of_memory_is_torchs_error():
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2 ** 20) / total)
+    held = []
     try:
+        while True:   # what earlier tests left free inside the reserved segments
+            try:
+                held.append(torch.empty(2 ** 25, dtype=torch.uint8, device=DEV))
+            except torch.OutOfMemoryError:
+                break
         with pytest.raises(torch.OutOfMemoryError):
             switch_gqa_prefill_forward(q, k, v, full, local)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+        held.clear()
     o, _ = switch_gqa_prefill_forward(q, k, v, full, local)
     assert bool(torch.isfinite(o).all())
 
