@@ -439,17 +439,18 @@ __device__ __forceinline__ void dkv_pair(const BwdParams& p, int r, int& t, int&
 // only against all of it; cutting finer starts more workgroups and writes and
 // reads back 256 KiB of partials for each.  In tenths of a us: a row block takes
 // 16, a dQ key tile 22 (a row tile has about one per two of its blocks' key
-// tiles), a workgroup's start and end 150, and a share of a cut pair 225 more, so
-//   16 c + 150 = per_cu + 225 (blocks / c) / CUs,
-// per_cu being the time per CU of the uncut grid.  (150 shapes of up to 4000
-// positions and 110 of up to 16384, backward, mean over the best of each: 0.8 and
-// 1.3 % with this, 3.4 and 3.2 % without the last term; the finest cut is 5 %
-// slower.)  The blocks are counted from the ranges: the host knows neither where
-// packed sequences end nor which positions are full.  (Taken from the list
-// lengths alone, 64 packed sequences of 128 keys and one of 8192, Hq8/Hkv2, took
-// 358 us, counted 234; eight of 300 to 1400 keys, Hq64/Hkv8, every row full, 550
-// and 263 us.)  The grid and the reduce must find the same value: no contraction,
-// and one float sum in one order.
+// tiles), a workgroup's start and end 150, and a share of a cut pair 375 more, so
+//   16 c + 150 = per_cu + 375 (blocks / c) / CUs,
+// per_cu being the time per CU of the uncut grid.  (Backward of 70 training shapes
+// and of 170 others of all kinds, mean over the best of several rules: 1.8 and
+// 2.2 % with this, 2.3 and 3.1 % with 225, 2.8 and 3.7 % with 900; on other such
+// sets 3.3 % without the last term and 5 % with the finest cut.)  The blocks are
+// counted from the ranges: the host knows neither where packed sequences end nor
+// which positions are full.  (Taken from the list lengths alone, 64 packed
+// sequences of 128 keys and one of 8192, Hq8/Hkv2, took 358 us, counted 234; eight
+// of 300 to 1400 keys, Hq64/Hkv8, every row full, 550 and 263 us.)  The grid and
+// the reduce must find the same value: no contraction, and one float sum in one
+// order.
 __device__ __forceinline__ float dkv_chunk(const BwdParams& p) {
 #pragma clang fp contract(off)
   const int lane = count_below(~uint64_t{0});
@@ -461,7 +462,7 @@ __device__ __forceinline__ float dkv_chunk(const BwdParams& p) {
   }
   blocks = wave_sum(blocks) * p.hkv;
   const float b = (27.f * blocks + 150.f * p.dkv_jobs) * (1.f / kDqSlots) - 150.f;
-  const float c = (b + __builtin_amdgcn_sqrtf(b * b + (64.f * 225.f / kDqSlots) * blocks)) * (1.f / 32);
+  const float c = (b + __builtin_amdgcn_sqrtf(b * b + (64.f * 375.f / kDqSlots) * blocks)) * (1.f / 32);
   return max(c, static_cast<float>(kDkvMinBlocks));
 }
 
@@ -537,24 +538,23 @@ __device__ __forceinline__ float4* part_unit(const BwdParams& p, int64_t wg, int
 }
 
 // dQ workgroup wg takes piece s of row tile t (full ones first) for KV head
-// kvh, KV head fastest: rows (tiles.h) of the full tiles, one per piece, the last
-// piece first, then rows of the local tiles.  Row tiles with more pieces are the
-// longer ones, so the grid runs by falling length but for the pieces' rounding.
-// dq_slot_wg is the inverse.
+// kvh, KV head fastest: rows (tiles.h) of the full tiles, one per piece, then rows
+// of the local tiles.  (The last piece first, as dK/dV's shares: 1 % slower in the
+// mean over 70 training shapes, 28 % at B1 S1215 Hq8/Hkv2, where rows of hardly
+// any piece then hold back the rest.)  dq_slot_wg is the inverse.
 __device__ __forceinline__ void dq_slot(const BwdParams& p, int wg, int& t, int& s, int& kvh) {
   kvh = wg % p.hkv;
   int x = wg / p.hkv;
   const int full_slots = p.items[0] * p.dq_maxc[0];
   const int b = x < full_slots ? 0 : 1;
   x -= b ? full_slots : 0;
-  const int row = x / p.items[b];
-  s = p.dq_maxc[b] - 1 - row;
-  t = (b ? p.items[0] : 0) + row_entry(x - row * p.items[b], row, p.items[b], p.hkv);
+  s = x / p.items[b];
+  t = (b ? p.items[0] : 0) + row_entry(x - s * p.items[b], s, p.items[b], p.hkv);
 }
 __device__ __forceinline__ int64_t dq_slot_wg(const BwdParams& p, int t, int s, int kvh) {
-  const int b = t < p.items[0] ? 0 : 1, row = p.dq_maxc[b] - 1 - s;
-  const int64_t x = static_cast<int64_t>(row) * p.items[b] +
-                    row_place(t - (b ? p.items[0] : 0), row, p.items[b], p.hkv);
+  const int b = t < p.items[0] ? 0 : 1;
+  const int64_t x = static_cast<int64_t>(s) * p.items[b] +
+                    row_place(t - (b ? p.items[0] : 0), s, p.items[b], p.hkv);
   return (x + (b ? static_cast<int64_t>(p.items[0]) * p.dq_maxc[0] : 0)) * p.hkv + kvh;
 }
 
@@ -1371,7 +1371,7 @@ __device__ __forceinline__ void dq_wide(const BwdParams& p, char* smem, int* s_r
 // dK/dV's last (longest) workgroups leave idle, and a small grid runs both at
 // once.  With that, pairs need cutting less often: at B2 S4096 Hq32/Hkv8 W1024
 // none is (307 us + 31 us of reduce + 225 us of dQ -> 524 us for both); B1
-// S1024 Hq8/Hkv2: 20.6 + 18.7 -> 22.6 us; B1 S16384 Hq32/Hkv8 1 % less.
+// S1024 Hq8/Hkv2: 20.6 + 18.7 -> 22.6 us; B1 S16384 Hq32/Hkv8 unchanged.
 constexpr int kWideLdsBytes = kDkvWideLdsBytes > kDqWideLdsBytes ? kDkvWideLdsBytes : kDqWideLdsBytes;
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void bwd_wide_kernel(const BwdParams p) {
