@@ -447,7 +447,7 @@ __device__ __forceinline__ void dkv_pair(const BwdParams& p, int r, int& t, int&
 // sets 3.3 % without the last term and 5 % with the finest cut.)  The blocks are
 // counted from the ranges: the host knows neither where packed sequences end nor
 // which positions are full.  (Taken from the list lengths alone, 64 packed
-// sequences of 128 keys and one of 8192, Hq8/Hkv2, took 358 us, counted 234; eight
+// sequences of 128 keys and one of 8192, Hq8/Hkv2, took 358 us, counted 254; eight
 // of 300 to 1400 keys, Hq64/Hkv8, every row full, 550 and 263 us.)  The grid and
 // the reduce must find the same value: no contraction, and one float sum in one
 // order.
